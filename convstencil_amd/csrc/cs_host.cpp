@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <vector>
@@ -81,28 +82,13 @@ int default_kf(int ndim, int R, int top, int shape, bool fp64) {
   return std::min(top, R == 1 ? 6 : 3);
 }
 
-std::vector<Variant> joined(const Variant *(*a)(int *), const Variant *(*b)(int *)) {
-  int na = 0, nb = 0;
-  const Variant *x = a(&na), *y = b(&nb);
-  std::vector<Variant> v(x, x + na);
-  v.insert(v.end(), y, y + nb);
-  return v;
-}
-
-std::vector<Variant> joined3(const Variant *(*a)(int *), const Variant *(*b)(int *), const Variant *(*c)(int *)) {
-  std::vector<Variant> v = joined(a, b);
-  int nc = 0;
-  const Variant *z = c(&nc);
-  v.insert(v.end(), z, z + nc);
-  return v;
-}
-
-std::vector<Variant> joined4(const Variant *(*a)(int *), const Variant *(*b)(int *), const Variant *(*c)(int *),
-                             const Variant *(*d)(int *)) {
-  std::vector<Variant> v = joined3(a, b, c);
-  int nd = 0;
-  const Variant *z = d(&nd);
-  v.insert(v.end(), z, z + nd);
+std::vector<Variant> joined(std::initializer_list<const Variant *(*)(int *)> lists) {
+  std::vector<Variant> v;
+  for (auto f : lists) {
+    int n = 0;
+    const Variant *x = f(&n);
+    v.insert(v.end(), x, x + n);
+  }
   return v;
 }
 
@@ -113,9 +99,10 @@ const Variant *family(int ndim, int *cnt, int prec = CS_PREC_FP64) {
   if (ndim < 1 || ndim > 3) return nullptr;
   // the MFMA kernels, then the --breakdown ladder's FMA kernels
   static const std::vector<Variant> all[3] = {
-      joined3(cs::variants_1d_reg, cs::variants_1d_f64, cs::variants_1d_ablation),
-      joined4(cs::variants_2d_f64, cs::variants_2d_reg, cs::variants_2d_stream, cs::variants_2d_ablation),
-      joined4(cs::variants_3d_reg, cs::variants_3d_f64, cs::variants_3d_fma, cs::variants_3d_ablation)};
+      joined({cs::variants_1d_reg, cs::variants_1d_f64, cs::variants_1d_ablation}),
+      joined({cs::variants_2d_f64, cs::variants_2d_reg, cs::variants_2d_pipe_r1, cs::variants_2d_pipe_r3,
+              cs::variants_2d_stream, cs::variants_2d_ablation}),
+      joined({cs::variants_3d_reg, cs::variants_3d_f64, cs::variants_3d_fma, cs::variants_3d_ablation})};
   *cnt = (int)all[ndim - 1].size();
   return all[ndim - 1].data();
 }
@@ -156,8 +143,9 @@ const Variant *single_step(int nd, int R, int shape, const Variant *v) {
   // GStencil/s against 242 for the register single step)
   if (v->mf == 9 && nd == 3)
     if (const Variant *m = find_variant(nd, 8, R, shape, 1, 0, CS_PREC_FP64)) return m;
-  if ((v->mf == 6 || v->mf == 7) && !(nd == 2 && R > 1 && shape == cs::SHAPE_BOX))
+  if ((v->mf == 6 || v->mf == 7 || v->mf == 10) && !(nd == 2 && R > 1 && shape == cs::SHAPE_BOX))
     if (const Variant *m = find_variant(nd, 4, R, shape, 1, 0, CS_PREC_FP64)) return m;
+  if (v->mf == 10) return find_variant(nd, 7, R, shape, 1, 0, CS_PREC_FP64);
   return find_variant(nd, v->mf, R, shape, 1, 0, CS_PREC_FP64);
 }
 
@@ -166,9 +154,43 @@ const Variant *single_step(int nd, int R, int shape, const Variant *v) {
 // 825 GStencil/s at depth 4 against 635 at depth 8; 3072^2: 1136 against 1183).
 constexpr int64_t kRegSmallGrid = 2560LL * 2560LL;
 
+// Whether a variant can run a 2-D interior of nx columns (the level-pipelined kernels' strips
+// lie inside the interior).
+bool fits(const Variant *v, int64_t nx) { return v->mf != 10 || nx >= 64 * v->px; }
+
+// The variant that runs r steps left over by a main variant v; null where there is none.  The
+// level-pipelined kernels are compiled for a few depths only; the register-streaming kernels
+// fill in, except for the radius-3 box, where those spill (3 steps at once 195 GStencil/s, 2 + 1
+// steps 320).
+const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int r, int prec, int st) {
+  const Variant *u = find_variant(nd, v->mf, R, shape, r, 0, prec, st);
+  if (!u && prec == CS_PREC_FP64 && v->mf == 10 && !(R > 1 && shape == cs::SHAPE_BOX))
+    u = find_variant(nd, 7, R, shape, r, 0, prec);
+  return u;
+}
+
+// The level-pipelined kernel for a 2-D FP64 grid of ny x nx cells, or null where the
+// register-streaming (or, box radius 3, the MFMA) kernels are the faster ones.  Every chunk pays
+// 2 R KF warm-up rows, and the pipelined kernels fuse deeper, so they need the larger grid:
+// measured, us per step of 96-step runs, other / this family:
+//   box r1   2048^2 5.0 / 5.3,   600 x 8000 5.3 / 5.1,  3072^2 8.2 / 7.4,   4096^2 11.7 / 10.4
+//   star r1  2048^2 3.7 / 3.7,   3072^2 5.4 / 5.3,      4096^2 8.2 / 6.9,   10240^2 49.4 / 34.1
+//   star r3  3072^2 13.1 / 13.9, 4096^2 19.0 / 17.9,    8192^2 66.8 / 57.4
+//   box r3   3072^2 33.5 / 39.6, 4096^2 56.5 / 52.9,    5120^2 90.0 / 69.0, 8192^2 219 / 147
+// Depths below the family's own are left to the others (box r1 depth 8 10240^2: 52.9 / 55.5).
+const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t nx) {
+  const bool box = shape == cs::SHAPE_BOX;
+  const int depth = R == 1 ? (box ? 12 : 16) : box ? 4 : 8;
+  const int64_t least = R == 1 ? (box ? 5000000 : 8000000) : 14000000;
+  if (nx < 512 || ny * nx < least || (fusion_depth > 0 && fusion_depth != depth)) return nullptr;
+  return find_variant(2, 10, R, shape, depth, 0);
+}
+
 // The main variant of a plan: a forced id, else the preferred family's default depth (for
-// 2-D, `cells` = the interior cells of one grid, 0 when no single grid decides).
-const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, int tile_variant, int64_t cells = 0) {
+// 2-D, ny x nx = the interior of one grid, 0 when no single grid decides).
+const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, int tile_variant, int64_t ny = 0,
+                         int64_t nx = 0) {
+  const int64_t cells = nd == 2 ? ny * nx : 0;
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
   const Variant *v = nullptr;
   if (tile_variant > 0) {
@@ -176,7 +198,10 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
     // stencil of its radius: the taps outside the stencil get zero weights)
     v = find_variant(nd, 0, R, shape, 0, tile_variant, prec);
     if (!v) v = find_variant(nd, 0, R, cs::SHAPE_BOX, 0, tile_variant, prec);
+    if (v && !fits(v, nx)) v = nullptr;
   } else if (prec == CS_PREC_FP64) {
+    if (nd == 2) v = pick_pipe(R, shape, fusion_depth, ny, nx);
+    if (v) return v;
     // 1-D: the register-resident kernels (mf 6) at their deepest compiled fusion, else the
     // 4 x 4 x 4 blocks; 2-D: the register-streaming kernels (mf 7), else the dilated 8 x 8
     // blocks; 3-D: the fused register-streaming kernels (mf 9, radius 1), else the 8 x 8
@@ -231,10 +256,10 @@ cs_status select_variants(cs_plan *p) {
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
   const Variant *v = nullptr;
   if (p->opt.tile_variant > 0) {
-    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant);
+    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2]);
     if (!v) return CS_ERR_INVALID;
   } else if (prec == CS_PREC_FP64) {
-    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, 0, nd == 2 ? p->L.n[1] * p->L.n[2] : 0);
+    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, 0, p->L.n[1], p->L.n[2]);
   } else {
     const int tries[3][2] = {{p->shape, 2}, {cs::SHAPE_BOX, 2}, {cs::SHAPE_BOX, 0}};
     for (const auto &tr : tries) {
@@ -256,7 +281,7 @@ cs_status select_variants(cs_plan *p) {
                                   : v->kf == 1 ? v : find_variant(nd, v->mf, p->R, p->shape, 1, 0, prec, fam);
   if (!p->vone) return CS_ERR_UNSUPPORTED;
   p->vrem.assign(v->kf, nullptr);
-  for (int r = 1; r < v->kf; ++r) p->vrem[r] = find_variant(nd, v->mf, p->R, p->shape, r, 0, prec, fam);
+  for (int r = 1; r < v->kf; ++r) p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
   for (const Variant *u : {p->vmain, p->vone}) CS_HIP(u->prepare());
   for (const Variant *u : p->vrem)
     if (u) CS_HIP(u->prepare());
@@ -272,15 +297,15 @@ cs_status select_variants(cs_plan *p) {
     CS_HIP(hipMemcpy(p->bfrag, hb.data(), bytes, hipMemcpyHostToDevice));
     return CS_OK;
   }
-  // the FMA kernels (the ladder's, the 3-D mf 3 family and the register-streaming mf 7 and
-  // mf 9 families) read the dense weights (zero-padded to whole 64-entry rows); a plan of
-  // those whose single steps run on an MFMA kernel (mf 7: the 2-D 4 x 4 x 4 kernel, mf 9:
+  // the FMA kernels (the ladder's, the 3-D mf 3 family, the register-streaming mf 7 and mf 9
+  // families and the level-pipelined mf 10 family) read the dense weights (zero-padded to whole 64-entry rows); a plan of
+  // those whose single steps run on an MFMA kernel (mf 7 and 10: the 2-D 4 x 4 x 4 kernel, mf 9:
   // the 3-D 8 x 8 blocks) appends that kernel's B fragments
   p->frag_off = 0;
-  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9) {
+  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10) {
     std::vector<double> h((p->w.size() + 63) / 64 * 64, 0.0);
     std::copy(p->w.begin(), p->w.end(), h.begin());
-    if (v->mf == 7 && p->vone->mf == 4) {
+    if ((v->mf == 7 || v->mf == 10) && p->vone->mf == 4) {
       p->frag_off = (int64_t)h.size();
       h.resize(h.size() + (size_t)cs::bfrag_ksteps_2d_f64(4, p->R, p->shape) * 64);
       cs::build_bfrag_2d_f64(4, p->R, p->shape, p->w.data(), h.data() + p->frag_off);
@@ -316,8 +341,12 @@ cs_status select_variants(cs_plan *p) {
   return CS_OK;
 }
 
-cs_status launch_one(cs_plan *p, const Variant *v) {
-  const Geo g = make_geo(p->L, v);
+// One launch of v; `done` = physical steps of the state's ping-pong so far.
+cs_status launch_one(cs_plan *p, const Variant *v, int64_t done) {
+  Geo g = make_geo(p->L, v);
+  // step `done` reads the halo of buffer done & 1; with halos that differ, the level-pipelined
+  // kernels are told when that is not the buffer that holds the state
+  g.flip = p->halo_uniform ? 0 : (p->cur ^ done) & 1;
   const double *wts = (v->mf == 4 || v->mf == 8) && p->frag_off > 0 ? p->bfrag + p->frag_off : p->bfrag;
   CS_HIP(v->launch(p->buf[p->cur], p->buf[p->cur ^ 1], wts, g, p->stream));
   p->cur ^= 1;
@@ -325,15 +354,24 @@ cs_status launch_one(cs_plan *p, const Variant *v) {
   return CS_OK;
 }
 
+// Whether the plan's launches may fuse steps: with halos that differ between the buffers only
+// the level-pipelined kernels can (they read every level's halo from its own buffer).
+bool fuses(const cs_plan *p) { return p->halo_uniform || p->vmain->mf == 10; }
+
 // Launch sequence for `steps` physical steps.  With uniform halos, fused
 // launches are exact: take the main depth as often as it fits, then the largest
 // compiled depth that fits the rest.  Otherwise every launch is a single step so
 // that each step reads the halo of its own buffer, as the reference's ping-pong
-// does.
+// does -- or, where the main variant is a level-pipelined kernel, launches of that family
+// (all of even depth) and single steps for the rest.  After those the state must lie in
+// the buffer whose halo it has by then, as after single steps: each even launch moves it to the
+// other one, so their number has to be even.  Of an odd number the last that two smaller
+// ones can replace is split, and if none can be, the last becomes single steps.  The single
+// steps come last, when the state is back in its own buffer.
 void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *> *seq) {
   seq->clear();
   if (steps <= 0) return;
-  if (!p->halo_uniform || p->vmain->kf == 1) {
+  if (!fuses(p) || p->vmain->kf == 1) {
     seq->assign((size_t)steps, p->vone);
     return;
   }
@@ -343,16 +381,50 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
   while (rem > 0) {
     const Variant *best = p->vone;
     for (const Variant *u : p->vrem)
-      if (u && u->kf <= rem && u->kf > best->kf) best = u;
+      if (u && u->kf <= rem && u->kf > best->kf && (p->halo_uniform || u->mf == 10)) best = u;
     seq->push_back(best);
     rem -= best->kf;
   }
+  if (p->vmain->mf == 10 && steps > kf && steps % kf) {
+    // a shallow last launch moves as many bytes as a deep one: kf + r steps are better cut
+    // evenly (box r1 10240^2, 12 + 4 against 8 + 8 steps: 0.91 against 0.84 ms)
+    const int r = (int)(steps % kf);
+    for (int b = (kf + r) / 2; b > r; --b) {
+      const Variant *u = kf + r - b < kf ? p->vrem[(size_t)(kf + r - b)] : nullptr, *v = p->vrem[(size_t)b];
+      if (!u || !v || (!p->halo_uniform && (u->mf != 10 || v->mf != 10))) continue;
+      seq->resize((size_t)(steps / kf) - 1);
+      seq->push_back(u);
+      seq->push_back(v);
+      break;
+    }
+  }
+  if (p->halo_uniform) return;
+  size_t n = 0;  // launches of the family come first
+  while (n < seq->size() && (*seq)[n]->mf == 10) ++n;
+  if (n % 2 == 0) return;
+  for (size_t i = n; i-- > 0;) {
+    const int k = (*seq)[i]->kf;
+    for (int half = k / 2; half >= 1; --half) {
+      const Variant *u = p->vrem[(size_t)half], *v = p->vrem[(size_t)(k - half)];
+      if (!u || !v || u->mf != 10 || v->mf != 10) continue;
+      (*seq)[i] = v;
+      seq->insert(seq->begin() + (ptrdiff_t)n, u);
+      return;
+    }
+  }
+  const int k = (*seq)[n - 1]->kf;
+  seq->erase(seq->begin() + (ptrdiff_t)(n - 1));
+  seq->insert(seq->end(), (size_t)k, p->vone);
 }
 
 cs_status issue_steps(cs_plan *p, int64_t steps) {
   std::vector<const Variant *> seq;
   plan_sequence(p, steps, &seq);
-  for (const Variant *v : seq) CS_TRY(launch_one(p, v));
+  int64_t done = p->steps_done;
+  for (const Variant *v : seq) {
+    CS_TRY(launch_one(p, v, done));
+    done += v->kf;
+  }
   return CS_OK;
 }
 
@@ -445,6 +517,7 @@ std::vector<const Variant *> tune_candidates(const cs_plan *p, int classified_sh
     // the --breakdown ladder's FMA kernels (for split plans mf holds the precision instead)
     if (p->opt.precision == CS_PREC_FP64 && (v.mf == 1 || v.mf == 2)) continue;
     if (p->opt.fusion_depth > 0 && v.kf != p->opt.fusion_depth) continue;
+    if (p->ndim == 2 && !fits(&v, p->L.n[2])) continue;
     out.push_back(&v);
   }
   return out;
@@ -570,13 +643,13 @@ namespace cs {
 // The FP64 kernel choice of a plan, made without a plan (nothing allocated, no device
 // touched): the main variant, the single-step variant and one variant per remainder depth
 // 1 .. kf - 1 (vrem[r], null where the family has none), as select_variants picks them for
-// a grid of `cells` interior cells.
+// a grid of ny x nx interior cells.
 // The launch sequence of the register-streaming 2-D family for `steps` steps of a radius-R
 // stencil of this shape class: the plan's default depth as often as it fits, then the
 // family's largest depth that fits the rest; empty when the plan would not take the family.
 void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> *seq) {
   seq->clear();
-  const Variant *v = pick_main(2, R, shape, CS_PREC_FP64, 0, 0);
+  const Variant *v = pick_main(2, R, shape, CS_PREC_FP64, 0, 0);  // no single grid: never mf 10
   if (!v || v->mf != 7) return;
   for (int64_t done = 0; done < steps;) {
     const int64_t rem = steps - done;
@@ -596,16 +669,16 @@ void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> 
   }
 }
 
-cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int tile_variant, int64_t cells,
+cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int tile_variant, int64_t ny, int64_t nx,
                              const Variant **vmain, const Variant **vone, const Variant **vrem, int vrem_cap) {
-  const Variant *v = pick_main(ndim, R, shape, CS_PREC_FP64, fusion_depth, tile_variant, cells);
+  const Variant *v = pick_main(ndim, R, shape, CS_PREC_FP64, fusion_depth, tile_variant, ny, nx);
   if (!v) return tile_variant > 0 ? CS_ERR_INVALID : CS_ERR_UNSUPPORTED;
   if (v->kf > vrem_cap) return CS_ERR_UNSUPPORTED;
   *vmain = v;
   *vone = single_step(ndim, R, v->shape, v);
   if (!*vone) return CS_ERR_UNSUPPORTED;
   for (int r = 0; r < vrem_cap; ++r)
-    vrem[r] = r >= 1 && r < v->kf ? find_variant(ndim, v->mf, R, v->shape, r, 0, CS_PREC_FP64) : nullptr;
+    vrem[r] = r >= 1 && r < v->kf ? remainder_variant(ndim, R, v->shape, v, r, CS_PREC_FP64, -1) : nullptr;
   return CS_OK;
 }
 
@@ -749,7 +822,7 @@ cs_status cs_plan_run(cs_plan *p, int64_t steps, cs_report *rep) {
   if (rep) {
     memset(rep, 0, sizeof(*rep));
     rep->launches = p->launches - l0;
-    rep->fusion_depth = p->halo_uniform ? p->vmain->kf : 1;
+    rep->fusion_depth = fuses(p) ? p->vmain->kf : 1;
     rep->variant = p->vmain->id;
   }
   return CS_OK;
@@ -782,7 +855,7 @@ cs_status cs_plan_time(cs_plan *p, int64_t steps, int32_t warmup, int32_t reps, 
     // a grid without interior cells launches nothing: no rate
     rep->gstencil_per_s = rep->elapsed_ms > 0 && pts > 0 ? pts * (double)steps / (rep->elapsed_ms * 1e-3) / 1e9 : 0.0;
     rep->launches = (p->launches - l0) / reps;
-    rep->fusion_depth = p->halo_uniform ? p->vmain->kf : 1;
+    rep->fusion_depth = fuses(p) ? p->vmain->kf : 1;
     rep->variant = p->vmain->id;
   }
   return CS_OK;
@@ -841,7 +914,7 @@ cs_status cs_run(const cs_layout *layout, const cs_stencil *st, const double *ho
     const double pts = (double)layout->n[0] * (double)layout->n[1] * (double)layout->n[2];
     rep->gstencil_per_s = ms > 0 ? pts * (double)steps / (ms * 1e-3) / 1e9 : 0.0;
     rep->launches = p->launches - l0;
-    rep->fusion_depth = p->halo_uniform ? p->vmain->kf : 1;
+    rep->fusion_depth = fuses(p) ? p->vmain->kf : 1;
     rep->variant = p->vmain->id;
   }
   if (e0) (void)hipEventDestroy(e0);

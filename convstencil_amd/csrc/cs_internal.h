@@ -65,6 +65,7 @@ struct Geo {
   int64_t org[3];    // interior origin
   int64_t n[3];      // interior sizes
   int64_t tiles[3];  // tiles per axis for this launch
+  int64_t flip;      // level-pipelined 2-D kernels: 1 = level 0's halo is the output buffer's
 };
 
 // Prefetch of a tile into L2 for the persistent kernels: one 8-byte load per thread and
@@ -265,6 +266,8 @@ const Variant *variants_1d_f64(int *count);
 const Variant *variants_1d_reg(int *count);   // register-resident FP64 1-D (k1d_reg.hip; mf 6)
 const Variant *variants_2d_f64(int *count);
 const Variant *variants_2d_reg(int *count);     // register-streaming FP64 2-D, radius 1 (k2d_reg.hip; mf 7)
+const Variant *variants_2d_pipe_r1(int *count);  // level-pipelined FP64 2-D (k2d_pipe_body.h; mf 10)
+const Variant *variants_2d_pipe_r3(int *count);
 const Variant *variants_2d_stream(int *count);  // pipelined persistent 2-D FP64 (k2d_stream.hip)
 const Variant *variants_3d_f64(int *count);  // all 3-D FP64 variants: k3d2 (mf 8) first, then k3d (mf 4)
 const Variant *variants_3d_reg(int *count);  // register-streaming FP64 3-D single steps (k3d_reg.hip; mf 9)
