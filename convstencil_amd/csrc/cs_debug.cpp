@@ -22,6 +22,7 @@ static const cs::Variant *family(int32_t ndim, int *n) {
   if (ndim == 9) return cs::variants_3d_reg(n);
   if (ndim == 10) return cs::variants_2d_pipe_r1(n);
   if (ndim == 11) return cs::variants_2d_pipe_r3(n);
+  if (ndim == 12) return cs::variants_2d_block(n);
   return nullptr;
 }
 

@@ -101,6 +101,7 @@ const Variant *family(int ndim, int *cnt, int prec = CS_PREC_FP64) {
   static const std::vector<Variant> all[3] = {
       joined({cs::variants_1d_reg, cs::variants_1d_f64, cs::variants_1d_ablation}),
       joined({cs::variants_2d_f64, cs::variants_2d_reg, cs::variants_2d_pipe_r1, cs::variants_2d_pipe_r3,
+              cs::variants_2d_block,
               cs::variants_2d_stream, cs::variants_2d_ablation}),
       joined({cs::variants_3d_reg, cs::variants_3d_f64, cs::variants_3d_fma, cs::variants_3d_ablation})};
   *cnt = (int)all[ndim - 1].size();
@@ -146,6 +147,7 @@ const Variant *single_step(int nd, int R, int shape, const Variant *v) {
   if ((v->mf == 6 || v->mf == 7 || v->mf == 10) && !(nd == 2 && R > 1 && shape == cs::SHAPE_BOX))
     if (const Variant *m = find_variant(nd, 4, R, shape, 1, 0, CS_PREC_FP64)) return m;
   if (v->mf == 10) return find_variant(nd, 7, R, shape, 1, 0, CS_PREC_FP64);
+  if (v->mf == 11) return find_variant(nd, 11, R, shape, 1, 0, CS_PREC_FP64, v->st);
   return find_variant(nd, v->mf, R, shape, 1, 0, CS_PREC_FP64);
 }
 
@@ -156,14 +158,16 @@ constexpr int64_t kRegSmallGrid = 2560LL * 2560LL;
 
 // Whether a variant can run a 2-D interior of nx columns (the level-pipelined kernels' strips
 // lie inside the interior).
-bool fits(const Variant *v, int64_t nx) { return v->mf != 10 || nx >= 64 * v->px; }
+bool fits(const Variant *v, int64_t ny, int64_t nx) {
+  return (v->mf != 10 && v->mf != 11) || (nx >= 64 * v->px && (v->mf != 11 || ny >= v->by));
+}
 
 // The variant that runs r steps left over by a main variant v; null where there is none.  The
 // level-pipelined kernels are compiled for a few depths only; the register-streaming kernels
 // fill in, except for the radius-3 box, where those spill (3 steps at once 195 GStencil/s, 2 + 1
 // steps 320).
 const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int r, int prec, int st) {
-  const Variant *u = find_variant(nd, v->mf, R, shape, r, 0, prec, st);
+  const Variant *u = find_variant(nd, v->mf, R, shape, r, 0, prec, v->mf == 11 && prec == CS_PREC_FP64 ? v->st : st);
   if (!u && prec == CS_PREC_FP64 && v->mf == 10 && !(R > 1 && shape == cs::SHAPE_BOX))
     u = find_variant(nd, 7, R, shape, r, 0, prec);
   return u;
@@ -186,6 +190,35 @@ const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t
   return find_variant(2, 10, R, shape, depth, 0);
 }
 
+// The register-tile kernel (k2d_block.hip) of the least predicted time per step for a small 2-D
+// FP64 grid, or null.  A launch of depth kf takes about 4.5 us + c (1.2 + a kf) us, c = tiles per
+// CU (at least 1) and a = 0.55 / 0.93 us a step for 32 / 64 rows (box radius 1), 0.42 / 0.75 (star
+// radius 1), 3.1 (star radius 3, one workgroup per CU): fitted to depths 1-12 on 300 x 517 to
+// 3072^2, within 10%, and its choice within 5% of the fastest depth.  Larger grids go to the
+// streaming kernels: box radius 1 3072^2 7.6 us per step against 7.4, star radius 1 5.7 against 5.4,
+// star radius 3 2048^2 11.1 against 9.6.
+const Variant *pick_block(int R, int shape, int64_t ny, int64_t nx) {
+  const bool box = shape == cs::SHAPE_BOX;
+  if (R == 2 || (R == 3 && box) || ny * nx >= (box ? 5000000 : 8000000)) return nullptr;
+  int cnt = 0;
+  const Variant *vs = cs::variants_2d_block(&cnt), *best = nullptr;
+  double best_t = 1e300;
+  for (int i = 0; i < cnt; ++i) {
+    const Variant &v = vs[i];
+    if (v.R != R || v.shape != shape || !fits(&v, ny, nx)) continue;
+    const int64_t wo = v.bx - 2 * R * v.kf, to = v.by - 2 * R * v.kf;
+    const int64_t tiles = (1 + (nx - v.bx + wo - 1) / wo) * (1 + (ny - v.by + to - 1) / to);
+    if (R == 3 && tiles > 256) continue;
+    const double a = R == 3 ? 3.1 : box ? (v.st == 4 ? 0.55 : 0.93) : (v.st == 4 ? 0.42 : 0.75);
+    const double t = (4.5 + std::max(1.0, (double)tiles / 256) * (1.2 + a * v.kf)) / v.kf;
+    if (t < best_t) {
+      best_t = t;
+      best = &v;
+    }
+  }
+  return best ? find_variant(2, 11, R, shape, best->kf, best->id) : nullptr;
+}
+
 // The main variant of a plan: a forced id, else the preferred family's default depth (for
 // 2-D, ny x nx = the interior of one grid, 0 when no single grid decides).
 const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, int tile_variant, int64_t ny = 0,
@@ -198,9 +231,10 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
     // stencil of its radius: the taps outside the stencil get zero weights)
     v = find_variant(nd, 0, R, shape, 0, tile_variant, prec);
     if (!v) v = find_variant(nd, 0, R, cs::SHAPE_BOX, 0, tile_variant, prec);
-    if (v && !fits(v, nx)) v = nullptr;
+    if (v && nd == 2 && prec == CS_PREC_FP64 && !fits(v, ny, nx)) v = nullptr;
   } else if (prec == CS_PREC_FP64) {
     if (nd == 2) v = pick_pipe(R, shape, fusion_depth, ny, nx);
+    if (nd == 2 && !v && fusion_depth == 0) v = pick_block(R, shape, ny, nx);
     if (v) return v;
     // 1-D: the register-resident kernels (mf 6) at their deepest compiled fusion, else the
     // 4 x 4 x 4 blocks; 2-D: the register-streaming kernels (mf 7), else the dilated 8 x 8
@@ -302,10 +336,10 @@ cs_status select_variants(cs_plan *p) {
   // those whose single steps run on an MFMA kernel (mf 7 and 10: the 2-D 4 x 4 x 4 kernel, mf 9:
   // the 3-D 8 x 8 blocks) appends that kernel's B fragments
   p->frag_off = 0;
-  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10) {
+  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10 || v->mf == 11) {
     std::vector<double> h((p->w.size() + 63) / 64 * 64, 0.0);
     std::copy(p->w.begin(), p->w.end(), h.begin());
-    if ((v->mf == 7 || v->mf == 10) && p->vone->mf == 4) {
+    if ((v->mf == 7 || v->mf == 10 || v->mf == 11) && p->vone->mf == 4) {
       p->frag_off = (int64_t)h.size();
       h.resize(h.size() + (size_t)cs::bfrag_ksteps_2d_f64(4, p->R, p->shape) * 64);
       cs::build_bfrag_2d_f64(4, p->R, p->shape, p->w.data(), h.data() + p->frag_off);
@@ -355,8 +389,11 @@ cs_status launch_one(cs_plan *p, const Variant *v, int64_t done) {
 }
 
 // Whether the plan's launches may fuse steps: with halos that differ between the buffers only
-// the level-pipelined kernels can (they read every level's halo from its own buffer).
-bool fuses(const cs_plan *p) { return p->halo_uniform || p->vmain->mf == 10; }
+// the level-pipelined and the register-tile kernels can (they read every level's halo from its
+// own buffer).
+bool fuses(const cs_plan *p) {
+  return p->halo_uniform || (p->opt.precision == CS_PREC_FP64 && (p->vmain->mf == 10 || p->vmain->mf == 11));
+}
 
 // Launch sequence for `steps` physical steps.  With uniform halos, fused
 // launches are exact: take the main depth as often as it fits, then the largest
@@ -376,6 +413,24 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
     return;
   }
   const int kf = p->vmain->kf;
+  if (p->opt.precision == CS_PREC_FP64 && p->vmain->mf == 11) {
+    // every depth is compiled: as few launches as the main depth allows, cut evenly.  With halos
+    // that differ an odd number of even depths k has one of them cut into k - 1 and 1.
+    const int64_t n = (steps + kf - 1) / kf;
+    int64_t even = 0;
+    for (int64_t i = 0; i < n; ++i) {
+      const int64_t d = steps / n + (i < steps % n);
+      seq->push_back(d == kf ? p->vmain : p->vrem[(size_t)d]);
+      even += d % 2 == 0;
+    }
+    if (!p->halo_uniform && even % 2) {
+      size_t i = 0;
+      while ((*seq)[i]->kf % 2) ++i;
+      (*seq)[i] = p->vrem[(size_t)(*seq)[i]->kf - 1];
+      seq->push_back(p->vone);
+    }
+    return;
+  }
   seq->assign((size_t)(steps / kf), p->vmain);
   int64_t rem = steps % kf;
   while (rem > 0) {
@@ -385,7 +440,7 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
     seq->push_back(best);
     rem -= best->kf;
   }
-  if (p->vmain->mf == 10 && steps > kf && steps % kf) {
+  if (p->opt.precision == CS_PREC_FP64 && p->vmain->mf == 10 && steps > kf && steps % kf) {
     // a shallow last launch moves as many bytes as a deep one: kf + r steps are better cut
     // evenly (box r1 10240^2, 12 + 4 against 8 + 8 steps: 0.91 against 0.84 ms)
     const int r = (int)(steps % kf);
@@ -517,7 +572,9 @@ std::vector<const Variant *> tune_candidates(const cs_plan *p, int classified_sh
     // the --breakdown ladder's FMA kernels (for split plans mf holds the precision instead)
     if (p->opt.precision == CS_PREC_FP64 && (v.mf == 1 || v.mf == 2)) continue;
     if (p->opt.fusion_depth > 0 && v.kf != p->opt.fusion_depth) continue;
-    if (p->ndim == 2 && !fits(&v, p->L.n[2])) continue;
+    if (p->ndim == 2 && p->opt.precision == CS_PREC_FP64 &&
+        (!fits(&v, p->L.n[1], p->L.n[2]) || (v.mf == 11 && p->L.n[1] * p->L.n[2] > 16000000)))
+      continue;  // the register tiles are for small grids
     out.push_back(&v);
   }
   return out;

@@ -268,6 +268,7 @@ const Variant *variants_2d_f64(int *count);
 const Variant *variants_2d_reg(int *count);     // register-streaming FP64 2-D, radius 1 (k2d_reg.hip; mf 7)
 const Variant *variants_2d_pipe_r1(int *count);  // level-pipelined FP64 2-D (k2d_pipe_body.h; mf 10)
 const Variant *variants_2d_pipe_r3(int *count);
+const Variant *variants_2d_block(int *count);  // a tile in a workgroup's registers, FP64 2-D (k2d_block.hip; mf 11)
 const Variant *variants_2d_stream(int *count);  // pipelined persistent 2-D FP64 (k2d_stream.hip)
 const Variant *variants_3d_f64(int *count);  // all 3-D FP64 variants: k3d2 (mf 8) first, then k3d (mf 4)
 const Variant *variants_3d_reg(int *count);  // register-streaming FP64 3-D single steps (k3d_reg.hip; mf 9)

@@ -93,11 +93,11 @@ extern "C" cs_status cs_run_2d_noalloc(const cs_layout *layout, const cs_stencil
   const cs::Variant *vmain = nullptr, *vone = nullptr, *vrem[32] = {};
   CS_TRY(cs::pick_fp64_variants(2, R, shape, o.fusion_depth, o.tile_variant, layout->n[1], layout->n[2],
                                 &vmain, &vone, vrem, 32));
-  // the dilated tables (mf 4: B fragments) and the register-streaming and level-pipelined
-  // kernels (mf 7, 10: dense weights, their single steps on the mf 4 kernel as in a plan):
+  // the dilated tables (mf 4: B fragments) and the register-streaming, level-pipelined
+  // and register-tile kernels (mf 7, 10, 11: dense weights, their single steps on the mf 4 kernel as in a plan):
   // scratch holds the dense weights first when the main variant is one of those, then the B
   // fragments when an mf 4 kernel runs
-  const bool dense = vmain->mf == 7 || vmain->mf == 10, frags4 = vmain->mf == 4 || vone->mf == 4;
+  const bool dense = vmain->mf == 7 || vmain->mf == 10 || vmain->mf == 11, frags4 = vmain->mf == 4 || vone->mf == 4;
   if (vmain->mf != 4 && !dense) return CS_ERR_UNSUPPORTED;
   const int D = 2 * R + 1;
   const int nks = frags4 ? cs::bfrag_ksteps_2d_f64(4, R, vmain->shape) : 0;
