@@ -23,6 +23,7 @@ static const cs::Variant *family(int32_t ndim, int *n) {
   if (ndim == 10) return cs::variants_2d_pipe_r1(n);
   if (ndim == 11) return cs::variants_2d_pipe_r3(n);
   if (ndim == 12) return cs::variants_2d_block(n);
+  if (ndim == 13) return cs::variants_3d_tile(n);
   return nullptr;
 }
 

@@ -103,7 +103,7 @@ const Variant *family(int ndim, int *cnt, int prec = CS_PREC_FP64) {
       joined({cs::variants_2d_f64, cs::variants_2d_reg, cs::variants_2d_pipe_r1, cs::variants_2d_pipe_r3,
               cs::variants_2d_block,
               cs::variants_2d_stream, cs::variants_2d_ablation}),
-      joined({cs::variants_3d_reg, cs::variants_3d_f64, cs::variants_3d_fma, cs::variants_3d_ablation})};
+      joined({cs::variants_3d_reg, cs::variants_3d_tile, cs::variants_3d_f64, cs::variants_3d_fma, cs::variants_3d_ablation})};
   *cnt = (int)all[ndim - 1].size();
   return all[ndim - 1].data();
 }
@@ -140,9 +140,9 @@ int max_kf(int ndim, int mf, int R, int shape, int prec = CS_PREC_FP64, int st =
 // 8192^2 286 against 253; box2d3r keeps its own (246 against 204).
 const Variant *single_step(int nd, int R, int shape, const Variant *v) {
   if (v->kf == 1) return v;
-  // the fused 3-D register kernels: the 8 x 8 block single-step kernel (512^3: 258-268
+  // the fused 3-D register and tile kernels: the 8 x 8 block single-step kernel (512^3: 258-268
   // GStencil/s against 242 for the register single step)
-  if (v->mf == 9 && nd == 3)
+  if ((v->mf == 9 || v->mf == 12) && nd == 3)
     if (const Variant *m = find_variant(nd, 8, R, shape, 1, 0, CS_PREC_FP64)) return m;
   if ((v->mf == 6 || v->mf == 7 || v->mf == 10) && !(nd == 2 && R > 1 && shape == cs::SHAPE_BOX))
     if (const Variant *m = find_variant(nd, 4, R, shape, 1, 0, CS_PREC_FP64)) return m;
@@ -156,9 +156,10 @@ const Variant *single_step(int nd, int R, int shape, const Variant *v) {
 // 825 GStencil/s at depth 4 against 635 at depth 8; 3072^2: 1136 against 1183).
 constexpr int64_t kRegSmallGrid = 2560LL * 2560LL;
 
-// Whether a variant can run a 2-D interior of nx columns (the level-pipelined kernels' strips
-// lie inside the interior).
+// Whether a variant can run an interior of ny rows of nx columns (the level-pipelined kernels' strips
+// and the tiles of the register-tile and the stacked 3-D kernels lie inside the interior).
 bool fits(const Variant *v, int64_t ny, int64_t nx) {
+  if (v->mf == 12) return nx >= v->bx && ny >= v->by;
   return (v->mf != 10 && v->mf != 11) || (nx >= 64 * v->px && (v->mf != 11 || ny >= v->by));
 }
 
@@ -167,6 +168,13 @@ bool fits(const Variant *v, int64_t ny, int64_t nx) {
 // fill in, except for the radius-3 box, where those spill (3 steps at once 195 GStencil/s, 2 + 1
 // steps 320).
 const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int r, int prec, int st) {
+  if (prec == CS_PREC_FP64 && v->mf == 12) {  // the same tile's shallower variants
+    int cnt = 0;
+    const Variant *vs = cs::variants_3d_tile(&cnt);
+    for (int i = 0; i < cnt; ++i)
+      if (vs[i].shape == shape && vs[i].by == v->by && vs[i].nw == v->nw && vs[i].kf == r) return &vs[i];
+    return nullptr;
+  }
   const Variant *u = find_variant(nd, v->mf, R, shape, r, 0, prec, v->mf == 11 && prec == CS_PREC_FP64 ? v->st : st);
   if (!u && prec == CS_PREC_FP64 && v->mf == 10 && !(R > 1 && shape == cs::SHAPE_BOX))
     u = find_variant(nd, 7, R, shape, r, 0, prec);
@@ -219,10 +227,28 @@ const Variant *pick_block(int R, int shape, int64_t ny, int64_t nx) {
   return best ? find_variant(2, 11, R, shape, best->kf, best->id) : nullptr;
 }
 
-// The main variant of a plan: a forced id, else the preferred family's default depth (for
-// 2-D, ny x nx = the interior of one grid, 0 when no single grid decides).
+// The stacked-wave 3-D kernel (k3d_tile.hip) of the least predicted time per step, or null where no
+// tile fits (fewer than 64 columns or 24 rows): the other families lose on every grid measured
+// that one fits, from 2% (box 40 x 500 x 500) to 4.6 times (box 64^3 22 -> 4.9 us).
+const Variant *pick_tile3(int R, int shape, int64_t nz, int64_t ny, int64_t nx) {
+  int cnt = 0;
+  const Variant *vs = cs::variants_3d_tile(&cnt), *best = nullptr;
+  double best_t = 1e300;
+  for (int i = 0; i < cnt; ++i) {
+    if (vs[i].R != R || vs[i].shape != shape || nz < 1 || !fits(&vs[i], ny, nx)) continue;
+    const double t = cs::tile3_cost(vs[i], nz, ny, nx);
+    if (t < best_t) {
+      best_t = t;
+      best = &vs[i];
+    }
+  }
+  return best ? find_variant(3, 12, R, shape, best->kf, best->id) : nullptr;
+}
+
+// The main variant of a plan: a forced id, else the preferred family's default depth (nz x ny x nx
+// = the interior of one grid, 0 when no single grid decides).
 const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, int tile_variant, int64_t ny = 0,
-                         int64_t nx = 0) {
+                         int64_t nx = 0, int64_t nz = 0) {
   const int64_t cells = nd == 2 ? ny * nx : 0;
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
   const Variant *v = nullptr;
@@ -231,10 +257,11 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
     // stencil of its radius: the taps outside the stencil get zero weights)
     v = find_variant(nd, 0, R, shape, 0, tile_variant, prec);
     if (!v) v = find_variant(nd, 0, R, cs::SHAPE_BOX, 0, tile_variant, prec);
-    if (v && nd == 2 && prec == CS_PREC_FP64 && !fits(v, ny, nx)) v = nullptr;
+    if (v && nd >= 2 && prec == CS_PREC_FP64 && !fits(v, ny, nx)) v = nullptr;
   } else if (prec == CS_PREC_FP64) {
     if (nd == 2) v = pick_pipe(R, shape, fusion_depth, ny, nx);
     if (nd == 2 && !v && fusion_depth == 0) v = pick_block(R, shape, ny, nx);
+    if (nd == 3 && fusion_depth == 0) v = pick_tile3(R, shape, nz, ny, nx);
     if (v) return v;
     // 1-D: the register-resident kernels (mf 6) at their deepest compiled fusion, else the
     // 4 x 4 x 4 blocks; 2-D: the register-streaming kernels (mf 7), else the dilated 8 x 8
@@ -290,10 +317,11 @@ cs_status select_variants(cs_plan *p) {
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
   const Variant *v = nullptr;
   if (p->opt.tile_variant > 0) {
-    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2]);
+    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2],
+                  p->L.n[0]);
     if (!v) return CS_ERR_INVALID;
   } else if (prec == CS_PREC_FP64) {
-    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, 0, p->L.n[1], p->L.n[2]);
+    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, 0, p->L.n[1], p->L.n[2], p->L.n[0]);
   } else {
     const int tries[3][2] = {{p->shape, 2}, {cs::SHAPE_BOX, 2}, {cs::SHAPE_BOX, 0}};
     for (const auto &tr : tries) {
@@ -332,18 +360,19 @@ cs_status select_variants(cs_plan *p) {
     return CS_OK;
   }
   // the FMA kernels (the ladder's, the 3-D mf 3 family, the register-streaming mf 7 and mf 9
-  // families and the level-pipelined mf 10 family) read the dense weights (zero-padded to whole 64-entry rows); a plan of
-  // those whose single steps run on an MFMA kernel (mf 7 and 10: the 2-D 4 x 4 x 4 kernel, mf 9:
-  // the 3-D 8 x 8 blocks) appends that kernel's B fragments
+  // families, the level-pipelined mf 10 family and the tiles of mf 11 and 12) read the dense weights (zero-padded to whole 64-entry rows); a plan of
+  // those whose single steps run on an MFMA kernel (mf 7 and 10: the 2-D 4 x 4 x 4 kernel, mf 9
+  // and 12: the 3-D 8 x 8 blocks) appends that kernel's B fragments
   p->frag_off = 0;
-  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10 || v->mf == 11) {
+  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10 || v->mf == 11 ||
+      v->mf == 12) {
     std::vector<double> h((p->w.size() + 63) / 64 * 64, 0.0);
     std::copy(p->w.begin(), p->w.end(), h.begin());
     if ((v->mf == 7 || v->mf == 10 || v->mf == 11) && p->vone->mf == 4) {
       p->frag_off = (int64_t)h.size();
       h.resize(h.size() + (size_t)cs::bfrag_ksteps_2d_f64(4, p->R, p->shape) * 64);
       cs::build_bfrag_2d_f64(4, p->R, p->shape, p->w.data(), h.data() + p->frag_off);
-    } else if (v->mf == 9 && p->vone->mf == 8) {
+    } else if ((v->mf == 9 || v->mf == 12) && p->vone->mf == 8) {
       p->frag_off = (int64_t)h.size();
       h.resize(h.size() + (size_t)cs::bfrag_ksteps_3d2_f64(p->R, p->shape) * 64);
       cs::build_bfrag_3d2_f64(p->R, p->shape, p->w.data(), h.data() + p->frag_off);
@@ -413,14 +442,16 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
     return;
   }
   const int kf = p->vmain->kf;
-  if (p->opt.precision == CS_PREC_FP64 && p->vmain->mf == 11) {
-    // every depth is compiled: as few launches as the main depth allows, cut evenly.  With halos
-    // that differ an odd number of even depths k has one of them cut into k - 1 and 1.
+  if (p->opt.precision == CS_PREC_FP64 && (p->vmain->mf == 11 || p->vmain->mf == 12)) {
+    // every depth is compiled (mf 12: from 2 up): as few launches as the main depth allows, cut
+    // evenly.  With halos that differ an odd number of even depths k has one of them cut into k - 1
+    // and 1.
     const int64_t n = (steps + kf - 1) / kf;
     int64_t even = 0;
     for (int64_t i = 0; i < n; ++i) {
       const int64_t d = steps / n + (i < steps % n);
-      seq->push_back(d == kf ? p->vmain : p->vrem[(size_t)d]);
+      const Variant *u = d == kf ? p->vmain : p->vrem[(size_t)d];
+      seq->push_back(u ? u : p->vone);
       even += d % 2 == 0;
     }
     if (!p->halo_uniform && even % 2) {
@@ -572,7 +603,7 @@ std::vector<const Variant *> tune_candidates(const cs_plan *p, int classified_sh
     // the --breakdown ladder's FMA kernels (for split plans mf holds the precision instead)
     if (p->opt.precision == CS_PREC_FP64 && (v.mf == 1 || v.mf == 2)) continue;
     if (p->opt.fusion_depth > 0 && v.kf != p->opt.fusion_depth) continue;
-    if (p->ndim == 2 && p->opt.precision == CS_PREC_FP64 &&
+    if (p->ndim >= 2 && p->opt.precision == CS_PREC_FP64 &&
         (!fits(&v, p->L.n[1], p->L.n[2]) || (v.mf == 11 && p->L.n[1] * p->L.n[2] > 16000000)))
       continue;  // the register tiles are for small grids
     out.push_back(&v);

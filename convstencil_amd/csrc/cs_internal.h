@@ -272,6 +272,8 @@ const Variant *variants_2d_block(int *count);  // a tile in a workgroup's regist
 const Variant *variants_2d_stream(int *count);  // pipelined persistent 2-D FP64 (k2d_stream.hip)
 const Variant *variants_3d_f64(int *count);  // all 3-D FP64 variants: k3d2 (mf 8) first, then k3d (mf 4)
 const Variant *variants_3d_reg(int *count);  // register-streaming FP64 3-D single steps (k3d_reg.hip; mf 9)
+const Variant *variants_3d_tile(int *count);  // stacked-wave FP64 3-D, radius 1 (k3d_tile.hip; mf 12)
+double tile3_cost(const Variant &v, int64_t nz, int64_t ny, int64_t nx);  // one of those: predicted us per step
 const Variant *variants_3d2_f64(int *count);  // 8 x 8 block family only
 const Variant *variants_2d_split(int *count);
 const Variant *variants_2d_ablation(int *count);  // --breakdown rungs 1-2 (mf 1, 2; forced by id only)

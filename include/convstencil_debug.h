@@ -29,7 +29,8 @@ extern "C" {
  * planes in the load ring); 10, 11 = the level-pipelined 2-D FP64 kernels of radius 1 and 3
  * (info[1] = 10, info[6] = output columns per workgroup of 64 x info[9], info[7] = waves the levels
  * are dealt over); 12 = the register-tile 2-D FP64 kernels (info[1] = 11, info[5] x info[6] = the
- * tile, halo included). */
+ * tile, halo included); 13 = the stacked-wave 3-D FP64 kernels (info[1] = 12, info[5] x info[6] = the
+ * tile's rows and columns, halo included). */
 int32_t cs_debug_variant_count(int32_t ndim);
 /* info[0..11] = id, mfma shape (16 or 4), radius, shape class (0 box, 1 star), fusion depth,
  * tile rows, tile cols (1-D: tile length), waves, LDS bytes, LDS row pitch / buffer length
