@@ -315,6 +315,13 @@ cs_status select_variants(cs_plan *p) {
   // stencil's shape class, else its box variants (zero weights off the stencil), else the
   // Toeplitz form (st 0, box only).  The remainder launches come from the same form.
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
+  // The 49-point box in FP16 w3 and BF16x3 takes depth 6 (even depths give the same bits, see CfgS2):
+  // below it a launch is bound by its bytes and its tile's load.  Measured, us a step at depth 2 and
+  // 6 on 64 x 64 tiles and at depth 6 on 80 x 64: FP16 w3 300 x 517 5.14, 4.08, 4.52; 2048^2 16.7, 11.6,
+  // 12.3; 4096^2 54.5, 39.9, 38.2; 8192^2 194.7, 131.9, 124.4; BF16x3 (64 x 64) 300 x 517 5.62, 4.58;
+  // 8192^2 214.0, 166.6.
+  const bool deep = nd == 2 && p->R == 3 && p->shape == cs::SHAPE_BOX && p->opt.fusion_depth == 0 &&
+                    p->opt.tile_variant <= 0 && (prec == CS_PREC_FP16W3 || prec == CS_PREC_BF16X3);
   const Variant *v = nullptr;
   if (p->opt.tile_variant > 0) {
     v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2],
@@ -329,6 +336,11 @@ cs_status select_variants(cs_plan *p) {
       if (top == 0) continue;
       int kf = p->opt.fusion_depth > 0 ? std::min(p->opt.fusion_depth, top)
                                        : default_kf(nd, p->R, top, tr[0], false);
+      if (deep && tr[0] == cs::SHAPE_BOX && tr[1] == 2) {
+        kf = 6;
+        if (prec == CS_PREC_FP16W3 && p->L.n[1] * p->L.n[2] >= 12000000)
+          v = find_variant(nd, mf, 3, cs::SHAPE_BOX, 6, 1463406, prec);
+      }
       for (; kf >= 1 && !v; --kf) v = find_variant(nd, mf, p->R, tr[0], kf, 0, prec, tr[1]);
       if (v) break;
     }
@@ -343,7 +355,8 @@ cs_status select_variants(cs_plan *p) {
                                   : v->kf == 1 ? v : find_variant(nd, v->mf, p->R, p->shape, 1, 0, prec, fam);
   if (!p->vone) return CS_ERR_UNSUPPORTED;
   p->vrem.assign(v->kf, nullptr);
-  for (int r = 1; r < v->kf; ++r) p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
+  for (int r = 1; r < v->kf; ++r)
+    if (!deep || r == 1 || r % 2 == 0) p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
   for (const Variant *u : {p->vmain, p->vone}) CS_HIP(u->prepare());
   for (const Variant *u : p->vrem)
     if (u) CS_HIP(u->prepare());

@@ -68,9 +68,20 @@ struct CfgS2 {
     for (int s = 0; s < KF; ++s) m = lox(s, cs) + CT.cmin < m ? lox(s, cs) + CT.cmin : m;
     return m;
   }
+  // An output's FP32 sum order depends on its place in its 2 x 8 anchor.  The 49-point box's deeper
+  // even depths put the anchors where depth 2 has them in the grid (rows: 2 R steps keep their
+  // parity; columns: KF R + CS mod 8), and a step's FP32 recombination rounds as FP64 state
+  // rounded to FP32 on load does: they give the bits of depth 2.
+  static constexpr int anchor() {
+    if constexpr (R == 3 && SH == SHAPE_BOX && KF > 2 && KF % 2 == 0) {
+      using Two = CfgS2<Tr_, R_, SH_, 2, 64, 64, 8>;
+      return (2 * R + Two::CS) % 8;
+    }
+    return -1;
+  }
   static constexpr int find_cs() {
     for (int cs = 0; cs < 64; ++cs)
-      if (min_col(cs) + cs >= 0) return cs;
+      if (min_col(cs) + cs >= 0 && (anchor() < 0 || (KF * R + cs) % 8 == anchor())) return cs;
     return 64;
   }
   static constexpr int CS = find_cs();
@@ -363,7 +374,8 @@ __device__ __forceinline__ void split_lane_setup(const typename C::T *__restrict
 }
 
 // Block origins of every fused step, per wave, as for the FP64 kernels (k2d_f64_body.h,
-// Org4): o = LDS byte offset of the block's first cell, yx = (y << 16) | x.
+// Org4): o = LDS byte offset of the block's first cell, yx = y in the upper half, x (which a block left
+// of the tile has below zero) in the lower one.
 template <class C>
 struct OrgS {
   static constexpr int base(int s) {
@@ -386,7 +398,7 @@ constexpr OrgS<C> make_orgs() {
         int y = 0, x = 0;
         C::origin(s, blk, y, x);
         t.o[w][OrgS<C>::base(s) + j] = (y * C::PX + x) * (int)sizeof(typename C::T);
-        t.yx[w][OrgS<C>::base(s) + j] = (y << 16) | x;
+        t.yx[w][OrgS<C>::base(s) + j] = (y << 16) | (x & 0xffff);
       }
   return t;
 }
@@ -449,15 +461,20 @@ __device__ __forceinline__ void split_step(const SplitCtx &t, const typename C::
   for (int j = 0; j < PERS; ++j) {
     if constexpr (!LAST) {
       Q q[C::NSU];
-      const float f[4] = {d0[j][0] + d1[j][0] * INV, d0[j][1] + d1[j][1] * INV, d0[j][2] + d1[j][2] * INV,
-                          d0[j][3] + d1[j][3] * INV};
+      float f[4] = {d0[j][0] + d1[j][0] * INV, d0[j][1] + d1[j][1] * INV, d0[j][2] + d1[j][2] * INV,
+                    d0[j][3] + d1[j][3] * INV};
+      if constexpr (C::anchor() >= 0 && S % 2 == 1) {
+        // the end of a depth-2 launch: rounded to FP32 by itself, not in one with the slice
+#pragma unroll
+        for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(f[e]));
+      }
       split4<Tr>(f, q);
       char *dst = lds + ot[j] + t.vw;
       if constexpr (!MASK) {
 #pragma unroll
         for (int k = 0; k < C::NSU; ++k) *reinterpret_cast<Q *>(dst + k * SB) = q[k];
       } else {
-        const int yx = yt[j], ty = (yx >> 16) + t.orow, tx0 = (yx & 0xffff) + t.ocol;
+        const int yx = yt[j], ty = (yx >> 16) + t.orow, tx0 = (short)(yx & 0xffff) + t.ocol;
         const bool row_in = (unsigned)(ty - t.ry0) < (unsigned)t.nry;
         if (row_in && (unsigned)(tx0 - t.cx0) < (unsigned)t.ncx && (unsigned)(tx0 + 3 - t.cx0) < (unsigned)t.ncx) {
 #pragma unroll
@@ -471,7 +488,7 @@ __device__ __forceinline__ void split_step(const SplitCtx &t, const typename C::
         }
       }
     } else {
-      const int yx = yt[j], y = yx >> 16, x = yx & 0xffff, ty = y + t.orow, tx0 = x + t.ocol;
+      const int yx = yt[j], y = yx >> 16, x = (short)(yx & 0xffff), ty = y + t.orow, tx0 = x + t.ocol;
       if constexpr (C::OS == 1) {
         // staged: the output block cell (ty - LO, tx - LO) of a compact BY x BX FP64 array
         double *ob = reinterpret_cast<double *>(lds) + (ty - C::LO(S)) * C::BX + tx0 - C::LO(S);
