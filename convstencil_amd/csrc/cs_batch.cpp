@@ -1,7 +1,8 @@
 // cs_batch.cpp -- host side of the batched workload (cs_batch_* in convstencil.h).
 //
-// FP64 batches whose grids all carry a uniform halo run on the register-streaming 2-D
-// kernels (k2d_reg.hip): launch j of the run advances every grid whose launch sequence
+// FP64 batches whose grids all carry a uniform halo run on the register-tile 2-D kernels
+// (k2d_block.hip), grids too small for a tile on the register-streaming ones
+// (k2d_reg.hip): launch j of the run advances every grid whose launch sequence
 // has a j-th launch, all grids of one kernel variant in one multi-grid launch (the kernel
 // boundary orders the steps; no device-wide barrier).  Every other batch runs the
 // persistent kernel: `steps` time steps of every grid become step blocks of work items
@@ -11,6 +12,7 @@
 #include <algorithm>
 #include <map>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/convstencil_debug.h"
@@ -83,6 +85,8 @@ struct cs_batch {
 
 namespace cs {
 void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> *seq);
+cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, int64_t>> &sizes, int64_t steps,
+                         std::vector<const Variant *> *seq);
 }
 
 namespace {
@@ -168,17 +172,25 @@ void free_rseq(RegSeq &s) {
   s = RegSeq{};
 }
 
-// Waves of grid g for variant v: strips of v's output columns cut into chunks of about 64
-// rows (the checked chunks shorter), as the single-grid launch cuts them.  Measured on the
+// Items of grid g for variant v.  Tiles (mf 11): every tile of the grid.  Else waves: strips of v's
+// output columns cut into chunks of about `rows` rows (the checked chunks shorter), as the single-grid launch cuts them.  Measured on the
 // batch of 256 grids (FP64, GStencil/s): 224-row chunks 513, 128 622, 64 662, 40 639 --
 // many short waves balance the launches' tails better than the warm-up rows they add.
-void reg_items(const cs_batch *b, int g, const cs::Variant *v, std::vector<cs::RegItem> *out) {
+void reg_items(const cs_batch *b, int g, const cs::Variant *v, int64_t rows, std::vector<cs::RegItem> *out) {
   const cs_layout &L = b->layouts[(size_t)g];
   const int64_t ny = L.n[1], nx = L.n[2];
   if (ny <= 0 || nx <= 0) return;
+  if (v->mf == 11) {
+    const int64_t wo = v->bx - 2 * v->R * v->kf, to = v->by - 2 * v->R * v->kf;
+    const int64_t tx = 1 + (nx - v->bx + wo - 1) / wo, ty = 1 + (ny - v->by + to - 1) / to;
+    for (int64_t y = 0; y < ty; ++y)
+      for (int64_t x = 0; x < tx; ++x)
+        out->push_back(cs::RegItem{g, (int)x, (int)y, (int)(x == tx - 1) | (int)(y == ty - 1) << 1});
+    return;
+  }
   const int ox = v->bx, h = v->R * v->kf;
   const int64_t strips = (nx + ox - 1) / ox;
-  const int64_t slots = strips * std::max<int64_t>(1, (ny + 63) / 64);
+  const int64_t slots = strips * std::max<int64_t>(1, (ny + rows - 1) / rows);
   const cs::RegSplit sp = cs::reg_split(ny, nx, ox, h, slots, cs::reg_edge_cost(v->px, v->R),
                                          cs::reg_least(v->R, v->kf, v->st));
   const int64_t waves = cs::reg_waves(sp);
@@ -188,50 +200,86 @@ void reg_items(const cs_batch *b, int g, const cs::Variant *v, std::vector<cs::R
   }
 }
 
+// A stencil class of at most this many cells takes tiles: a launch of the streaming kernels lasts as long as
+// its chains of rows, a tile's overlap costs FMAs.  Measured, us per step, streaming / tiles: 16 box
+// grids of 4.8 M cells 11.3 / 5.8, 8 star grids of 2.9 M cells (two of them too narrow for a tile) 15.9 /
+// 13.3; 256 grids of 118 M cells 143 / 259.
+constexpr int64_t kTileCells = 8000000;
+
+int64_t cells(const std::vector<std::pair<int64_t, int64_t>> &sizes) {
+  int64_t n = 0;
+  for (const auto &s : sizes) n += s.first * s.second;
+  return n;
+}
+
 // The register path's launches for `steps` steps: launch j groups, per variant, every grid
 // whose sequence has a j-th launch.
 cs_status build_rseq(cs_batch *b, int64_t steps, RegSeq *s) {
   std::vector<std::vector<const cs::Variant *>> seq((size_t)b->count);
   std::vector<int> chain((size_t)b->count);
-  std::vector<std::pair<int, int>> classes;  // (R, shape) in order of first appearance
-  size_t nj = 0;
+  // (radius, shape class, takes tiles) in order of first appearance
+  typedef std::tuple<int, int, bool> Class;
+  std::vector<Class> classes;
+  std::vector<std::vector<std::pair<int64_t, int64_t>>> sizes;
   for (int g = 0; g < b->count; ++g) {
-    const std::pair<int, int> c(b->R[(size_t)g], b->shape[(size_t)g]);
+    const int R = b->R[(size_t)g];
+    const cs_layout &L = b->layouts[(size_t)g];
+    // the tiles' least: 32 x 128 cells at radius 1, 64 x 256 at radius 3
+    const Class c(R, b->shape[(size_t)g], L.n[1] >= (R == 1 ? 32 : 64) && L.n[2] >= (R == 1 ? 128 : 256));
     size_t k = 0;
     while (k < classes.size() && classes[k] != c) ++k;
-    if (k == classes.size()) classes.push_back(c);
+    if (k == classes.size()) {
+      classes.push_back(c);
+      sizes.emplace_back();
+    }
     chain[(size_t)g] = (int)k;
-    cs::reg_sequence(b->R[(size_t)g], b->shape[(size_t)g], steps, &seq[(size_t)g]);
+    sizes[k].emplace_back(L.n[1], L.n[2]);
+  }
+  std::vector<std::vector<const cs::Variant *>> tiles(classes.size());
+  for (size_t k = 0; k < classes.size(); ++k)
+    if (std::get<2>(classes[k]) && cells(sizes[k]) <= kTileCells)
+      CS_TRY(cs::block_sequence(std::get<0>(classes[k]), std::get<1>(classes[k]), sizes[k], steps, &tiles[k]));
+  // streamed classes: 64-row chunks, shorter ones (down to 16 rows) where those make fewer waves than
+  // the chip has SIMDs, since a launch then lasts as long as one chunk
+  std::vector<int64_t> rows(classes.size());
+  for (size_t k = 0; k < classes.size(); ++k) {
+    int64_t waves = 0;
+    for (const auto &n : sizes[k]) waves += (n.second + 127) / 128 * ((n.first + 63) / 64);
+    rows[k] = std::min<int64_t>(64, std::max<int64_t>(16, 64 * waves / 1024));
+  }
+  size_t nj = 0;
+  for (int g = 0; g < b->count; ++g) {
+    seq[(size_t)g] = tiles[(size_t)chain[(size_t)g]];
+    if (seq[(size_t)g].empty()) cs::reg_sequence(b->R[(size_t)g], b->shape[(size_t)g], steps, &seq[(size_t)g]);
     if (seq[(size_t)g].empty()) return CS_ERR_UNSUPPORTED;
     nj = std::max(nj, seq[(size_t)g].size());
     s->parity_flip.push_back((int)(seq[(size_t)g].size() & 1));
   }
   std::map<std::pair<int, const cs::Variant *>, std::vector<cs::RegItem>> cache;
   for (size_t j = 0; j < nj; ++j) {
-    std::map<const cs::Variant *, std::vector<cs::RegItem>> groups;
-    std::map<const cs::Variant *, int> group_chain;
+    // per variant and chain: a chain's launches keep its stream
+    std::map<std::pair<const cs::Variant *, int>, std::vector<cs::RegItem>> groups;
     for (int g = 0; g < b->count; ++g) {
       if (j >= seq[(size_t)g].size()) continue;
       const cs::Variant *v = seq[(size_t)g][j];
-      group_chain[v] = chain[(size_t)g];  // a variant serves one stencil class
       auto key = std::make_pair(g, v);
       auto c = cache.find(key);
       if (c == cache.end()) {
         std::vector<cs::RegItem> it;
-        reg_items(b, g, v, &it);
+        reg_items(b, g, v, rows[(size_t)chain[(size_t)g]], &it);
         c = cache.emplace(key, it).first;
       }
-      std::vector<cs::RegItem> &dst = groups[v];
+      std::vector<cs::RegItem> &dst = groups[std::make_pair(v, chain[(size_t)g])];
       dst.insert(dst.end(), c->second.begin(), c->second.end());
     }
     for (auto &kv : groups) {
       if (kv.second.empty()) continue;
       if (kv.second.size() > (size_t)0x7fffffff) return CS_ERR_UNSUPPORTED;
       RegLaunch l;
-      l.v = kv.first;
+      l.v = kv.first.first;
       l.nitems = (int)kv.second.size();
       l.flip = (int)(j & 1);
-      l.chain = group_chain[kv.first];
+      l.chain = kv.first.second;
       CS_HIP(hipMalloc(&l.items, kv.second.size() * sizeof(cs::RegItem)));
       s->launches.push_back(l);  // freed with the sequence from here on
       CS_HIP(hipMemcpy(l.items, kv.second.data(), kv.second.size() * sizeof(cs::RegItem), hipMemcpyHostToDevice));

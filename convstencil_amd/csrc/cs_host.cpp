@@ -198,6 +198,14 @@ const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t
   return find_variant(2, 10, R, shape, depth, 0);
 }
 
+// Predicted us per step of a launch of the register-tile kernel v over `tiles` tiles (see pick_block).
+double block_cost(const Variant &v, int64_t tiles) {
+  const bool box = v.shape == cs::SHAPE_BOX;
+  const double a = v.R == 3 ? 3.1 : box ? (v.st == 4 ? 0.55 : 0.93) : (v.st == 4 ? 0.42 : 0.75);
+  const double c = v.R == 3 ? (double)((tiles + 255) / 256) : std::max(1.0, (double)tiles / 256);
+  return (4.5 + c * (1.2 + a * v.kf)) / v.kf;
+}
+
 // The register-tile kernel (k2d_block.hip) of the least predicted time per step for a small 2-D
 // FP64 grid, or null.  A launch of depth kf takes about 4.5 us + c (1.2 + a kf) us, c = tiles per
 // CU (at least 1) and a = 0.55 / 0.93 us a step for 32 / 64 rows (box radius 1), 0.42 / 0.75 (star
@@ -217,8 +225,7 @@ const Variant *pick_block(int R, int shape, int64_t ny, int64_t nx) {
     const int64_t wo = v.bx - 2 * R * v.kf, to = v.by - 2 * R * v.kf;
     const int64_t tiles = (1 + (nx - v.bx + wo - 1) / wo) * (1 + (ny - v.by + to - 1) / to);
     if (R == 3 && tiles > 256) continue;
-    const double a = R == 3 ? 3.1 : box ? (v.st == 4 ? 0.55 : 0.93) : (v.st == 4 ? 0.42 : 0.75);
-    const double t = (4.5 + std::max(1.0, (double)tiles / 256) * (1.2 + a * v.kf)) / v.kf;
+    const double t = block_cost(v, tiles);
     if (t < best_t) {
       best_t = t;
       best = &v;
@@ -768,6 +775,44 @@ void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> 
     seq->push_back(u);
     done += u->kf;
   }
+}
+
+// The same for the register-tile kernels, for several grids of one stencil that share their launches
+// (sizes: rows, columns): empty when there is no tile that fits them all.  A launch of depth kf takes what
+// pick_block says, with the tiles of all grids (radius 3, one workgroup per CU: whole rounds).
+cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, int64_t>> &sizes, int64_t steps,
+                         std::vector<const Variant *> *seq) {
+  seq->clear();
+  int cnt = 0;
+  const Variant *vs = variants_2d_block(&cnt), *best = nullptr;
+  double best_t = 1e300;
+  for (int i = 0; i < cnt; ++i) {
+    const Variant &v = vs[i];
+    if (v.R != R || v.shape != shape || v.kf > steps) continue;
+    const int64_t wo = v.bx - 2 * R * v.kf, to = v.by - 2 * R * v.kf;
+    int64_t tiles = 0;
+    bool ok = !sizes.empty();
+    for (const auto &n : sizes) {
+      ok = ok && fits(&v, n.first, n.second);
+      if (ok) tiles += (1 + (n.second - v.bx + wo - 1) / wo) * (1 + (n.first - v.by + to - 1) / to);
+    }
+    if (!ok) continue;
+    const double t = block_cost(v, tiles);
+    if (t < best_t) {
+      best_t = t;
+      best = &v;
+    }
+  }
+  if (!best) return CS_OK;
+  const int64_t n = (steps + best->kf - 1) / best->kf;
+  for (int64_t i = 0; i < n; ++i) {
+    const int64_t d = steps / n + (i < steps % n);
+    const Variant *u = find_variant(2, 11, R, shape, (int)d, 0, CS_PREC_FP64, best->st);
+    if (!u) return CS_ERR_UNSUPPORTED;
+    CS_HIP(u->prepare());
+    seq->push_back(u);
+  }
+  return CS_OK;
 }
 
 cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int tile_variant, int64_t ny, int64_t nx,

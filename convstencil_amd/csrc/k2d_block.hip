@@ -233,18 +233,18 @@ __device__ __forceinline__ void run_block(const double *in, double *out, const d
   t.run(kf, ys, left, right);
 }
 
+extern __shared__ __attribute__((aligned(16))) double block_lds[];
+
+// Tile (by, bx) of a grid by kf steps; right, bottom: the last one of its axis.
 template <int R, int SHAPE, int PX, int BR, int NWV>
-__global__ __launch_bounds__(NWV * 64, R == 1 ? 4 : 2) void k2d_block(const double *in, double *out, const double *wts, Geo g,
-                                                     BlockSplit sp) {
+__device__ __forceinline__ void block_tile(const double *in, double *out, const double *wts, const Geo &g, int kf,
+                                           int bx, int by, bool right, bool bottom) {
   using C = Block2D<R, PX, BR, NWV>;
-  extern __shared__ __attribute__((aligned(16))) double block_lds[];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int by = __builtin_amdgcn_readfirstlane(blockIdx.x / (unsigned)sp.tx);
-  const int bx = (int)blockIdx.x - by * sp.tx;
-  const int H = R * sp.kf;
+  const int H = R * kf;
   const int64_t ny = g.n[1], nx = g.n[2], pitch = g.ext[2];
-  const bool left = bx == 0, right = bx == sp.tx - 1, top = by == 0, bottom = by == sp.ty - 1;
+  const bool left = bx == 0, top = by == 0;
   const int64_t xs = right ? nx - C::W : (int64_t)bx * (C::W - 2 * H);
   const int64_t ys = bottom ? ny - C::TR : (int64_t)by * (C::TR - 2 * H);
   bool general = false;
@@ -273,10 +273,28 @@ __global__ __launch_bounds__(NWV * 64, R == 1 ? 4 : 2) void k2d_block(const doub
     general = __syncthreads_or(any != 0);
   }
   if (general)
-    run_block<R, SHAPE, PX, BR, NWV, true>(in, out, wts, g, sp.kf, xs, ys, left, right, top, bottom, lane, wv, block_lds);
+    run_block<R, SHAPE, PX, BR, NWV, true>(in, out, wts, g, kf, xs, ys, left, right, top, bottom, lane, wv, block_lds);
   else
-    run_block<R, SHAPE, PX, BR, NWV, false>(in, out, wts, g, sp.kf, xs, ys, left, right, top, bottom, lane, wv,
+    run_block<R, SHAPE, PX, BR, NWV, false>(in, out, wts, g, kf, xs, ys, left, right, top, bottom, lane, wv,
                                             block_lds);
+}
+
+template <int R, int SHAPE, int PX, int BR, int NWV>
+__global__ __launch_bounds__(NWV * 64, R == 1 ? 4 : 2) void k2d_block(const double *in, double *out, const double *wts, Geo g,
+                                                     BlockSplit sp) {
+  const int by = __builtin_amdgcn_readfirstlane(blockIdx.x / (unsigned)sp.tx);
+  const int bx = (int)blockIdx.x - by * sp.tx;
+  block_tile<R, SHAPE, PX, BR, NWV>(in, out, wts, g, sp.kf, bx, by, bx == sp.tx - 1, by == sp.ty - 1);
+}
+
+// The tiles of several grids: item.strip, item.y0 = bx, by; item.y1 = right | bottom << 1.
+template <int R, int SHAPE, int PX, int BR, int NWV>
+__global__ __launch_bounds__(NWV * 64, R == 1 ? 4 : 2) void k2d_block_multi(RegMulti mm, int kf) {
+  const RegItem it = mm.items[blockIdx.x];
+  const RegGrid *G = mm.grids + it.grid;
+  const int cur = G->cur ^ mm.flip;
+  block_tile<R, SHAPE, PX, BR, NWV>(G->buf[cur], G->buf[cur ^ 1], G->wts, G->geo, kf, it.strip, it.y0, it.y1 & 1,
+                                    it.y1 >> 1);
 }
 
 template <int R, int SHAPE, int PX, int BR, int NWV>
@@ -285,8 +303,18 @@ struct BlockLaunch {
   static constexpr size_t kLds = C::LDS * sizeof(double);
 
   static hipError_t prepare() {
-    return hipFuncSetAttribute((const void *)k2d_block<R, SHAPE, PX, BR, NWV>,
+    hipError_t e = hipFuncSetAttribute((const void *)k2d_block<R, SHAPE, PX, BR, NWV>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
+    if (e != hipSuccess) return e;
+    return hipFuncSetAttribute((const void *)k2d_block_multi<R, SHAPE, PX, BR, NWV>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
+  }
+
+  template <int KF>
+  static hipError_t launch_multi(const RegMulti &mm, hipStream_t s) {
+    hipLaunchKernelGGL((k2d_block_multi<R, SHAPE, PX, BR, NWV>), dim3((unsigned)mm.nitems), dim3(NWV * 64), kLds, s, mm,
+                       KF);
+    return hipGetLastError();
   }
 
   template <int KF>
@@ -310,7 +338,8 @@ struct BlockLaunch {
   Variant {                                                                                                  \
     ID + KF, 11, R, SH, KF, NWV *BR, 64 * PX, NWV, BlockLaunch<R, SH, PX, BR, NWV>::kLds, PX, BR,            \
         &BlockLaunch<R, SH, PX, BR, NWV>::launch<KF>, &BlockLaunch<R, SH, PX, BR, NWV>::prepare,             \
-        "k2d_block<r" #R "," #SH ",p" #PX "," #BR "x" #NWV ",kf" #KF ">"                                     \
+        "k2d_block<r" #R "," #SH ",p" #PX "," #BR "x" #NWV ",kf" #KF ">",                                    \
+        0, &BlockLaunch<R, SH, PX, BR, NWV>::launch_multi<KF>                                                \
   }
 #define CS_VB2D7(ID, R, SH, PX, BR, NWV)                                            \
   CS_VB2D(ID, R, SH, PX, BR, NWV, 1), CS_VB2D(ID, R, SH, PX, BR, NWV, 2),           \
