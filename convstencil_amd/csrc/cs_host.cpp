@@ -938,7 +938,8 @@ cs_status cs_plan_upload(cs_plan *p, const double *host_in) {
   p->cur = 0;
   p->steps_done = 0;
   p->halo_uniform = halo_is_zero(&p->L, host_in);
-  p->amax = abs_max(host_in, n);
+  // the scan (5.2 ms for 2048^2, of 11 ms for a whole host-to-host run) serves the FP16 range guard only
+  p->amax = p->opt.precision == CS_PREC_FP16X2 || p->opt.precision == CS_PREC_FP16W3 ? abs_max(host_in, n) : 0.0;
   return CS_OK;
 }
 
