@@ -479,23 +479,31 @@ template <int R, int SH, int PX, int KFW, int NWV, int B, int NSB, int RING>
 struct PipeVariant {
   using C = Pipe2D<R, PX, KFW, NWV, B>;
   static constexpr size_t kLds = C::LDS * sizeof(double);
-  static std::atomic<int64_t> slots;  // resident workgroups on this device
+  // resident workgroups on each device, 0 where prepare() has not run: the LDS attribute belongs to
+  // one device's copy of the kernel
+  static constexpr int kDevices = 64;
+  static std::atomic<int64_t> slots[kDevices];
 
   static hipError_t prepare() {
-    if (slots.load(std::memory_order_relaxed) > 0) return hipSuccess;
-    const void *f = (const void *)k2d_pipe<R, SH, PX, KFW, NWV, B, NSB, RING>;
-    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
-    if (e != hipSuccess) return e;
     int nb = 0, dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const bool known = dev >= 0 && dev < kDevices;
+    if (known && slots[dev].load(std::memory_order_relaxed) > 0) return hipSuccess;
+    const void *f = (const void *)k2d_pipe<R, SH, PX, KFW, NWV, B, NSB, RING>;
+    if ((e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds)) != hipSuccess) return e;
     if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, NWV * 64, kLds)) != hipSuccess) return e;
-    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-    slots.store((int64_t)(nb > 0 ? nb : 1) * (cus > 0 ? cus : 1), std::memory_order_relaxed);
+    if (known) slots[dev].store((int64_t)(nb > 0 ? nb : 1) * (cus > 0 ? cus : 1), std::memory_order_relaxed);
     return hipSuccess;
   }
 
   static hipError_t launch(const double *in, double *out, const double *wts, const Geo &g, hipStream_t s) {
-    const int64_t ny = g.n[1], nx = g.n[2], n = slots.load(std::memory_order_relaxed);
+    int dev = 0;
+    const hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const int64_t ny = g.n[1], nx = g.n[2];
+    const int64_t n = dev >= 0 && dev < kDevices ? slots[dev].load(std::memory_order_relaxed) : 0;
     if (nx < C::W || ny < 1) return hipErrorInvalidValue;  // strips are 64 PX columns of the interior
     PipeSplit sp;
     const int64_t strips = 1 + (nx - C::W + C::OX - 1) / C::OX;
@@ -514,7 +522,7 @@ struct PipeVariant {
 };
 
 template <int R, int SH, int PX, int KFW, int NWV, int B, int NSB, int RING>
-std::atomic<int64_t> PipeVariant<R, SH, PX, KFW, NWV, B, NSB, RING>::slots{0};
+std::atomic<int64_t> PipeVariant<R, SH, PX, KFW, NWV, B, NSB, RING>::slots[kDevices] = {};
 
 }  // namespace
 

@@ -1,0 +1,66 @@
+// hip_stub.cpp -- a HIP runtime that launches nothing, for host-code tests without a GPU: two gfx950
+// devices, and a launch with more than 64 KiB of dynamic LDS fails unless the kernel's attribute
+// was raised on the device that is current, as each device holds a kernel's attributes of its own.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstring>
+#include <map>
+#include <utility>
+
+namespace {
+int g_dev = 0, g_launches = 0, g_refused = 0;
+std::map<std::pair<int, const void *>, int> g_lds;
+double g_scratch[2][4096];
+hipError_t g_last = hipSuccess;
+struct Call {
+  dim3 grid, block;
+  size_t lds;
+  hipStream_t stream;
+} g_call;
+}  // namespace
+
+extern "C" {
+int stub_launches() { return g_launches; }
+int stub_refused() { return g_refused; }
+
+hipError_t hipGetDeviceCount(int *n) { return *n = 2, hipSuccess; }
+hipError_t hipGetDevice(int *d) { return *d = g_dev, hipSuccess; }
+hipError_t hipSetDevice(int d) { return g_dev = d, hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {
+  memset(p, 0, sizeof(*p));
+  strcpy(p->gcnArchName, "gfx950:sramecc+:xnack-");
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipGetSymbolAddress(void **p, const void *) { return *p = g_scratch[g_dev], hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute a, int v) {
+  if (a == hipFuncAttributeMaxDynamicSharedMemorySize) g_lds[{g_dev, f}] = v;
+  return hipSuccess;
+}
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) { return *n = 2, hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) {
+  g_call = Call{g, b, lds, s};
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s) {
+  *g = g_call.grid, *b = g_call.block, *lds = g_call.lds, *s = g_call.stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t lds, hipStream_t) {
+  ++g_launches;
+  const auto it = g_lds.find({g_dev, f});
+  if (lds > 65536 && (it == g_lds.end() || (size_t)it->second < lds)) {
+    ++g_refused;
+    return g_last = hipErrorInvalidValue;
+  }
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
+const char *hipGetErrorString(hipError_t) { return "stub"; }
+}
