@@ -175,6 +175,8 @@ const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int
       if (vs[i].shape == shape && vs[i].by == v->by && vs[i].nw == v->nw && vs[i].kf == r) return &vs[i];
     return nullptr;
   }
+  if (prec != CS_PREC_FP64 && v->st == 3)  // the bits of depth 2: even depths, with its anchors above it
+    return r > 1 && r % 2 ? nullptr : find_variant(nd, v->mf, R, shape, r, 0, prec, r > 2 ? 3 : 2);
   const Variant *u = find_variant(nd, v->mf, R, shape, r, 0, prec, v->mf == 11 && prec == CS_PREC_FP64 ? v->st : st);
   if (!u && prec == CS_PREC_FP64 && v->mf == 10 && !(R > 1 && shape == cs::SHAPE_BOX))
     u = find_variant(nd, 7, R, shape, r, 0, prec);
@@ -322,7 +324,7 @@ cs_status select_variants(cs_plan *p) {
   // stencil's shape class, else its box variants (zero weights off the stencil), else the
   // Toeplitz form (st 0, box only).  The remainder launches come from the same form.
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
-  // The 49-point box in FP16 w3 and BF16x3 takes depth 6 (even depths give the same bits, see CfgS2):
+  // The 49-point box in FP16 w3 and BF16x3 takes depth 6 with the anchors of depth 2 (st 3, see CfgS2):
   // below it a launch is bound by its bytes and its tile's load.  Measured, us a step at depth 2 and
   // 6 on 64 x 64 tiles and at depth 6 on 80 x 64: FP16 w3 300 x 517 5.14, 4.08, 4.52; 2048^2 16.7, 11.6,
   // 12.3; 4096^2 54.5, 39.9, 38.2; 8192^2 194.7, 131.9, 124.4; BF16x3 (64 x 64) 300 x 517 5.62, 4.58;
@@ -343,18 +345,16 @@ cs_status select_variants(cs_plan *p) {
       if (top == 0) continue;
       int kf = p->opt.fusion_depth > 0 ? std::min(p->opt.fusion_depth, top)
                                        : default_kf(nd, p->R, top, tr[0], false);
-      if (deep && tr[0] == cs::SHAPE_BOX && tr[1] == 2) {
-        kf = 6;
-        if (prec == CS_PREC_FP16W3 && p->L.n[1] * p->L.n[2] >= 12000000)
-          v = find_variant(nd, mf, 3, cs::SHAPE_BOX, 6, 1463406, prec);
-      }
+      if (deep && tr[0] == cs::SHAPE_BOX && tr[1] == 2)
+        v = find_variant(nd, mf, 3, cs::SHAPE_BOX, 6,
+                         prec == CS_PREC_FP16W3 && p->L.n[1] * p->L.n[2] >= 12000000 ? 3263406 : 0, prec, 3);
       for (; kf >= 1 && !v; --kf) v = find_variant(nd, mf, p->R, tr[0], kf, 0, prec, tr[1]);
       if (v) break;
     }
   }
   if (!v) return CS_ERR_UNSUPPORTED;
   p->shape = v->shape;
-  const int fam = prec != CS_PREC_FP64 ? v->st : -1;
+  const int fam = prec == CS_PREC_FP64 ? -1 : v->st == 3 ? 2 : v->st;
   p->vmain = v;
   // single-step launches: the chosen variant itself when it is a single-step one (a variant
   // forced by id must be the one that runs), else the family's first single-step variant
@@ -363,14 +363,14 @@ cs_status select_variants(cs_plan *p) {
   if (!p->vone) return CS_ERR_UNSUPPORTED;
   p->vrem.assign(v->kf, nullptr);
   for (int r = 1; r < v->kf; ++r)
-    if (!deep || r == 1 || r % 2 == 0) p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
+    p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
   for (const Variant *u : {p->vmain, p->vone}) CS_HIP(u->prepare());
   for (const Variant *u : p->vrem)
     if (u) CS_HIP(u->prepare());
   if (prec != CS_PREC_FP64) {
     std::vector<unsigned char> hb(1 << 20);
     const size_t bytes = nd == 3      ? cs::build_bfrag_split3(prec, p->R, p->shape, p->w.data(), hb.data(), hb.size())
-                         : v->st == 2 ? cs::build_bfrag_split2(prec, p->R, p->shape, p->w.data(), hb.data(), hb.size())
+                         : v->st >= 2 ? cs::build_bfrag_split2(prec, p->R, p->shape, p->w.data(), hb.data(), hb.size())
                                       : cs::build_bfrag_split(prec, p->R, p->w.data(), hb.data(), hb.size());
     if (bytes == 0) return CS_ERR_UNSUPPORTED;
     if (p->bfrag) (void)hipFree(p->bfrag);

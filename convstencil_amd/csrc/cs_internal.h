@@ -254,7 +254,7 @@ struct Variant {
   size_t lds_bytes;
   int px;  // LDS row pitch in doubles
   int st;  // fused-step staging: 0 = two LDS buffers, 1 = one buffer + registers;
-           // split-precision: 0 = Toeplitz form, 2 = dilated form
+           // split-precision: 0 = Toeplitz form, 2 = dilated form, 3 = that with the anchors of depth 2
   LaunchFn launch;  // one launch = kf fused steps from `in` to `out`
   hipError_t (*prepare)();  // one-time function attributes (dynamic LDS above 64 KiB)
   const char *name;

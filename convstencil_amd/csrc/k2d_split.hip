@@ -17,7 +17,7 @@ __global__ __launch_bounds__(NW * 64) void k2d_split(const double *__restrict__ 
   tile_split<Tr, R, KF, BY, BX, NW>(in, out, bfrag, g, tile, smem, threadIdx.x);
 }
 
-template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int OS>
+template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int OS, int AN>
 __global__ __launch_bounds__(NW * 64) void k2d_split2(const double *__restrict__ in, double *__restrict__ out,
                                                       const typename Tr::T *__restrict__ bfrag, Geo g) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -25,22 +25,22 @@ __global__ __launch_bounds__(NW * 64) void k2d_split2(const double *__restrict__
   const int64_t per = (ntiles + 7) / 8;
   const int64_t tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (tile >= ntiles) return;
-  tile_split2<Tr, R, SH, KF, BY, BX, NW, 64, OS>(in, out, bfrag, g, tile, smem, threadIdx.x);
+  tile_split2<Tr, R, SH, KF, BY, BX, NW, 64, OS, AN>(in, out, bfrag, g, tile, smem, threadIdx.x);
 }
 
-template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int OS>
+template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int OS, int AN>
 static hipError_t prepare_ks2() {
-  using C = CfgS2<Tr, R, SH, KF, BY, BX, NW, OS>;
-  return hipFuncSetAttribute((const void *)k2d_split2<Tr, R, SH, KF, BY, BX, NW, OS>,
+  using C = CfgS2<Tr, R, SH, KF, BY, BX, NW, OS, AN>;
+  return hipFuncSetAttribute((const void *)k2d_split2<Tr, R, SH, KF, BY, BX, NW, OS, AN>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS);
 }
 
-template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int OS>
+template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int OS, int AN>
 static hipError_t launch_ks2(const double *in, double *out, const double *bfrag, const Geo &g, hipStream_t s) {
-  using C = CfgS2<Tr, R, SH, KF, BY, BX, NW, OS>;
+  using C = CfgS2<Tr, R, SH, KF, BY, BX, NW, OS, AN>;
   const int64_t ntiles = g.tiles[1] * g.tiles[2];
   const int64_t grid = ((ntiles + 7) / 8) * 8;
-  hipLaunchKernelGGL((k2d_split2<Tr, R, SH, KF, BY, BX, NW, OS>), dim3((unsigned)grid), dim3(NW * 64), C::LDS, s,
+  hipLaunchKernelGGL((k2d_split2<Tr, R, SH, KF, BY, BX, NW, OS, AN>), dim3((unsigned)grid), dim3(NW * 64), C::LDS, s,
                      in, out, reinterpret_cast<const typename Tr::T *>(bfrag), g);
   return hipGetLastError();
 }
@@ -162,15 +162,17 @@ static hipError_t launch_ks(const double *in, double *out, const double *bfrag, 
 
 // Dilated form: Variant::st = 2.  Ids 60000 + R * 1000 + precision * 100 + (star) * 10 + KF;
 // 700000 + that: staged output (OS = 1); 800000 + that: 128 x 64 tiles; 900000 + that:
-// 128 x 128 tiles with 16 waves.
-#define CS_VS2O(ID, PREC, TR, R, SH, KF, BY, BX, NW, OS)                                                \
+// 128 x 128 tiles with 16 waves.  Variant::st = 3, ids 1800000 + that: the anchors of depth 2.
+#define CS_VS2X(ID, PREC, TR, R, SH, KF, BY, BX, NW, OS, AN, ST, TAIL)                                          \
   Variant {                                                                                             \
-    ID, PREC, R, SH, KF, BY, BX, NW, CfgS2<TR, R, SH, KF, BY, BX, NW, OS>::LDS,                         \
-        CfgS2<TR, R, SH, KF, BY, BX, NW, OS>::PX, 2, &launch_ks2<TR, R, SH, KF, BY, BX, NW, OS>,       \
-        &prepare_ks2<TR, R, SH, KF, BY, BX, NW, OS>,                                                    \
-        "k2d_split2<" #TR ",r" #R "," #SH ",kf" #KF "," #BY "x" #BX ",w" #NW ",os" #OS ">",             \
-        CfgS2<TR, R, SH, KF, BY, BX, NW, OS>::CS                                                        \
+    ID, PREC, R, SH, KF, BY, BX, NW, CfgS2<TR, R, SH, KF, BY, BX, NW, OS, AN>::LDS,                         \
+        CfgS2<TR, R, SH, KF, BY, BX, NW, OS, AN>::PX, ST, &launch_ks2<TR, R, SH, KF, BY, BX, NW, OS, AN>,       \
+        &prepare_ks2<TR, R, SH, KF, BY, BX, NW, OS, AN>,                                                    \
+        "k2d_split2<" #TR ",r" #R "," #SH ",kf" #KF "," #BY "x" #BX ",w" #NW ",os" #OS TAIL,           \
+        CfgS2<TR, R, SH, KF, BY, BX, NW, OS, AN>::CS                                                        \
   }
+#define CS_VS2O(ID, PREC, TR, R, SH, KF, BY, BX, NW, OS) CS_VS2X(ID, PREC, TR, R, SH, KF, BY, BX, NW, OS, 0, 2, ">")
+#define CS_VS2A(ID, PREC, TR, R, SH, KF, BY, BX, NW) CS_VS2X(ID, PREC, TR, R, SH, KF, BY, BX, NW, 0, 1, 3, ",an1>")
 #define CS_VS2(ID, PREC, TR, R, SH, KF, BY, BX, NW) CS_VS2O(ID, PREC, TR, R, SH, KF, BY, BX, NW, 0)
 
 #define CS_VS2P(ID, PREC, TR, R, SH, KF, BY, BX, NW)                                                    \
@@ -265,6 +267,12 @@ static const Variant kVariantsSplit[] = {
     CS_VS2O(763304, 3, TrF16, 3, SHAPE_BOX, 4, 64, 64, 8, 1),
     CS_VS2O(763404, 4, TrF16W3, 3, SHAPE_BOX, 4, 64, 64, 8, 1),
     CS_VS2O(763406, 4, TrF16W3, 3, SHAPE_BOX, 6, 64, 64, 8, 1),
+    // the anchors of depth 2: what plans of the 49-point box take by themselves
+    CS_VS2A(1863106, 1, TrBF16, 3, SHAPE_BOX, 6, 64, 64, 8),
+    CS_VS2A(1863104, 1, TrBF16, 3, SHAPE_BOX, 4, 64, 64, 8),
+    CS_VS2A(1863406, 4, TrF16W3, 3, SHAPE_BOX, 6, 64, 64, 8),
+    CS_VS2A(1863404, 4, TrF16W3, 3, SHAPE_BOX, 4, 64, 64, 8),
+    CS_VS2A(3263406, 4, TrF16W3, 3, SHAPE_BOX, 6, 80, 64, 8),
     // persistent dilated form (ids 500000 + the id of the same configuration)
     CS_VS2P(561102, 1, TrBF16, 1, SHAPE_BOX, 2, 64, 64, 8),
     CS_VS2P(561104, 1, TrBF16, 1, SHAPE_BOX, 4, 64, 64, 8),

@@ -43,8 +43,8 @@ struct Quad<TrF16W3> {
 };
 
 // OS = 1: the last step's FP64 results are staged in LDS (over the slice planes, which
-// are no longer read) and written out row by row, coalesced.
-template <class Tr_, int R_, int SH_, int KF_, int BY_, int BX_, int NW_, int OS_ = 0>
+// are no longer read) and written out row by row, coalesced.  AN = 1: the anchors of depth 2 (below).
+template <class Tr_, int R_, int SH_, int KF_, int BY_, int BX_, int NW_, int OS_ = 0, int AN_ = 0>
 struct CfgS2 {
   using Tr = Tr_;
   using T = typename Tr::T;
@@ -68,12 +68,16 @@ struct CfgS2 {
     for (int s = 0; s < KF; ++s) m = lox(s, cs) + CT.cmin < m ? lox(s, cs) + CT.cmin : m;
     return m;
   }
-  // An output's FP32 sum order depends on its place in its 2 x 8 anchor.  The 49-point box's deeper
-  // even depths put the anchors where depth 2 has them in the grid (rows: 2 R steps keep their
-  // parity; columns: KF R + CS mod 8), and a step's FP32 recombination rounds as FP64 state
-  // rounded to FP32 on load does: they give the bits of depth 2.
+  // An output's FP32 sum order depends on its place in its 2 x 8 anchor.  With AN = 1 an even depth
+  // of the 49-point box puts the anchors where depth 2 has them in the grid (rows: 2 R steps keep
+  // their parity; columns: KF R + CS mod 8) and rounds a step's recombination to FP32 by itself, as
+  // FP64 state is rounded on load, so it gives the bits of depth 2 except where the FP64 sum of a
+  // depth-2 launch's last step is itself a tie between two FP32 numbers.  The wider columns cost
+  // 2-5% (box2d3r 8192^2, depth 6, us a step: FP16 w3 125.5 -> 127.6), so only the kernels that plans
+  // take by themselves carry them; a depth asked for or tuned takes the others.
   static constexpr int anchor() {
-    if constexpr (R == 3 && SH == SHAPE_BOX && KF > 2 && KF % 2 == 0) {
+    if constexpr (AN_ != 0) {
+      static_assert(R == 3 && SH == SHAPE_BOX && KF > 2 && KF % 2 == 0, "anchors of depth 2");
       using Two = CfgS2<Tr_, R_, SH_, 2, 64, 64, 8>;
       return (2 * R + Two::CS) % 8;
     }
@@ -546,11 +550,11 @@ __device__ __forceinline__ void run_split_steps(const SplitCtx &t, const typenam
 // One workgroup advances tile `tile` of grid g by KF steps (smem: the kernel's dynamic
 // LDS; bfrag: the weights' slices as A fragments; LG: tile loads in flight per thread
 // for tiles at the domain edge; tid: threadIdx.x).
-template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int LG = 64, int OS = 0>
+template <class Tr, int R, int SH, int KF, int BY, int BX, int NW, int LG = 64, int OS = 0, int AN = 0>
 __device__ __forceinline__ void tile_split2(const double *__restrict__ in, double *__restrict__ out,
                                             const typename Tr::T *__restrict__ bfrag, const Geo &g, int64_t tile,
                                             unsigned char *__restrict__ smem, int tid) {
-  using C = CfgS2<Tr, R, SH, KF, BY, BX, NW, OS>;
+  using C = CfgS2<Tr, R, SH, KF, BY, BX, NW, OS, AN>;
   using T = typename Tr::T;
   using V = typename Tr::V;
   T *lds = reinterpret_cast<T *>(smem);
