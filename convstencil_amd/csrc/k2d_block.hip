@@ -28,6 +28,8 @@ namespace {
 
 typedef const double __attribute__((address_space(4))) cdouble;  // scalar loads
 typedef const double __attribute__((address_space(1))) gdouble;
+typedef const RegItem __attribute__((address_space(4))) citem;
+typedef const RegGrid __attribute__((address_space(4))) cgrid;
 typedef double pair_t __attribute__((ext_vector_type(2)));
 
 struct BlockSplit {
@@ -46,7 +48,7 @@ __device__ __forceinline__ double upper_or(double v, double f) {
   return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ uint64_t opaque(const double *p) {
+__device__ __forceinline__ uint64_t opaque(const void *p) {
   const uint64_t v = (uint64_t)p;
   uint64_t u = (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)v) |
                ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
@@ -128,7 +130,9 @@ struct BlockRun {
       }
     }
     lds_barrier();
-    const double *hb = ((s + flip) & 1) ? out : in;  // the buffer whose halo this step reads
+    // the buffer whose halo this step reads; a choice between copies, as in k2d_pipe_body.h (halo_buffer)
+    const double *const even = in, *const odd = out;
+    const double *hb = ((s + flip) & 1) ? odd : even;
 #pragma unroll
     for (int i = -R; i < BR + R; ++i) {
       double q[PX], qe[PX + 2 * R];
@@ -216,7 +220,7 @@ __device__ __forceinline__ void run_block(const double *in, double *out, const d
   t.in = in;
   t.out = out;
 #pragma unroll
-  for (int i = 0; i < t.D * t.D; ++i) t.w[i] = wts[i];
+  for (int i = 0; i < t.D * t.D; ++i) t.w[i] = ((cdouble *)opaque(wts))[i];
   t.pitch = g.ext[2];
   t.ey = g.ext[1];
   t.oy = g.org[1];
@@ -290,11 +294,21 @@ __global__ __launch_bounds__(NWV * 64, R == 1 ? 4 : 2) void k2d_block(const doub
 // The tiles of several grids: item.strip, item.y0 = bx, by; item.y1 = right | bottom << 1.
 template <int R, int SHAPE, int PX, int BR, int NWV>
 __global__ __launch_bounds__(NWV * 64, R == 1 ? 4 : 2) void k2d_block_multi(RegMulti mm, int kf) {
-  const RegItem it = mm.items[blockIdx.x];
-  const RegGrid *G = mm.grids + it.grid;
-  const int cur = G->cur ^ mm.flip;
-  block_tile<R, SHAPE, PX, BR, NWV>(G->buf[cur], G->buf[cur ^ 1], G->wts, G->geo, kf, it.strip, it.y0, it.y1 & 1,
-                                    it.y1 >> 1);
+  // item, grid and weights by scalar loads: they are the workgroup's, and as vectors they spill (radius
+  // 3: 66 registers)
+  const citem *it = (citem *)opaque(mm.items + blockIdx.x);
+  const cgrid *G = (cgrid *)opaque(mm.grids + it->grid);
+  const int cur = G->cur ^ mm.flip, y1 = it->y1;
+  Geo g;
+  for (int d = 0; d < 3; ++d) {
+    g.ext[d] = G->geo.ext[d];
+    g.org[d] = G->geo.org[d];
+    g.n[d] = G->geo.n[d];
+  }
+  g.flip = G->geo.flip;
+  const double *const b0 = G->buf[0], *const b1 = G->buf[1];
+  block_tile<R, SHAPE, PX, BR, NWV>(cur ? b1 : b0, (double *)(cur ? b0 : b1), G->wts, g, kf, it->strip, it->y0, y1 & 1,
+                                    y1 >> 1);
 }
 
 template <int R, int SHAPE, int PX, int BR, int NWV>
