@@ -6,6 +6,7 @@
 #include "cs_fused_weights.h"
 #include "cs_host_util.h"
 #include "cs_internal.h"
+#include "cs_sequence.h"
 
 extern "C" {
 
@@ -45,6 +46,21 @@ int32_t cs_debug_variant_info(int32_t ndim, int32_t i, int64_t *info, char *name
     name[len - 1] = 0;
   }
   return 0;
+}
+
+int32_t cs_debug_sequence_2d(int32_t radius, int32_t shape, int64_t ny, int64_t nx, int32_t zero_halo, int64_t steps,
+                             int32_t *ids, int64_t *counts, int32_t cap) {
+  cs::Sequence2D q;
+  if (steps < 1 || !ids || !counts || !q.init(radius, shape, ny, nx, zero_halo != 0)) return 0;
+  int n = 0;
+  q.each(steps, [&](const cs::Variant *v, int64_t count) {
+    if (n < cap) {
+      ids[n] = v->id;
+      counts[n] = count;
+    }
+    ++n;
+  });
+  return n > cap ? -1 : n;
 }
 
 int32_t cs_debug_ktable(int32_t mf, int32_t radius, int32_t shape, int32_t *dy, int32_t *c0, int32_t *live,

@@ -22,6 +22,7 @@
 #include "cs_host_util.h"
 #include "cs_internal.h"
 #include "cs_rng.h"
+#include "cs_sequence.h"
 
 using cs::Geo;
 using cs::Variant;
@@ -45,6 +46,9 @@ struct cs_plan {
   const Variant *vmain = nullptr;
   std::vector<const Variant *> vrem;  // vrem[r] runs r fused steps (r < vmain->kf), may be null
   const Variant *vone = nullptr;      // single-step variant (the register families use the MFMA one)
+  // 2-D FP64 plans that choose for themselves: the sequences for a zero halo [1] and another one [0]
+  bool by_time = false;
+  cs::Sequence2D seq[2];
   std::map<std::pair<int64_t, int>, hipGraphExec_t> graphs;
   int64_t launches = 0;
   int tuned = 0;  // 0 defaults or a forced variant, 1 cached autotuner choice, 2 timed now
@@ -183,57 +187,16 @@ const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int
   return u;
 }
 
-// The level-pipelined kernel for a 2-D FP64 grid of ny x nx cells, or null where the
-// register-streaming (or, box radius 3, the MFMA) kernels are the faster ones.  Every chunk pays
-// 2 R KF warm-up rows, and the pipelined kernels fuse deeper, so they need the larger grid:
-// measured, us per step of 96-step runs, other / this family:
-//   box r1   2048^2 5.0 / 5.3,   600 x 8000 5.3 / 5.1,  3072^2 8.2 / 7.4,   4096^2 11.7 / 10.4
-//   star r1  2048^2 3.7 / 3.7,   3072^2 5.4 / 5.3,      4096^2 8.2 / 6.9,   10240^2 49.4 / 34.1
-//   star r3  3072^2 13.1 / 13.9, 4096^2 19.0 / 17.9,    8192^2 66.8 / 57.4
-//   box r3   3072^2 33.5 / 39.6, 4096^2 56.5 / 52.9,    5120^2 90.0 / 69.0, 8192^2 219 / 147
-// Depths below the family's own are left to the others (box r1 depth 8 10240^2: 52.9 / 55.5).
+// The level-pipelined kernel of the depth that the caller asks for, the family's own, on a grid of a size
+// where it is the faster one (plans without a wish: cs_sequence.cpp), or null.  Measured, us per step
+// of 96-step runs, other / this family: box r1 2048^2 5.0 / 5.3, 3072^2 8.2 / 7.4; star r1 3072^2
+// 5.4 / 5.3; star r3 3072^2 13.1 / 13.9, 4096^2 19.0 / 17.9; box r3 3072^2 33.5 / 39.6, 4096^2 56.5 / 52.9.
 const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t nx) {
   const bool box = shape == cs::SHAPE_BOX;
   const int depth = R == 1 ? (box ? 12 : 16) : box ? 4 : 8;
   const int64_t least = R == 1 ? (box ? 5000000 : 8000000) : 14000000;
-  if (nx < 512 || ny * nx < least || (fusion_depth > 0 && fusion_depth != depth)) return nullptr;
+  if (nx < 512 || ny * nx < least || fusion_depth != depth) return nullptr;
   return find_variant(2, 10, R, shape, depth, 0);
-}
-
-// Predicted us per step of a launch of the register-tile kernel v over `tiles` tiles (see pick_block).
-double block_cost(const Variant &v, int64_t tiles) {
-  const bool box = v.shape == cs::SHAPE_BOX;
-  const double a = v.R == 3 ? 3.1 : box ? (v.st == 4 ? 0.55 : 0.93) : (v.st == 4 ? 0.42 : 0.75);
-  const double c = v.R == 3 ? (double)((tiles + 255) / 256) : std::max(1.0, (double)tiles / 256);
-  return (4.5 + c * (1.2 + a * v.kf)) / v.kf;
-}
-
-// The register-tile kernel (k2d_block.hip) of the least predicted time per step for a small 2-D
-// FP64 grid, or null.  A launch of depth kf takes about 4.5 us + c (1.2 + a kf) us, c = tiles per
-// CU (at least 1) and a = 0.55 / 0.93 us a step for 32 / 64 rows (box radius 1), 0.42 / 0.75 (star
-// radius 1), 3.1 (star radius 3, one workgroup per CU): fitted to depths 1-12 on 300 x 517 to
-// 3072^2, within 10%, and its choice within 5% of the fastest depth.  Larger grids go to the
-// streaming kernels: box radius 1 3072^2 7.6 us per step against 7.4, star radius 1 5.7 against 5.4,
-// star radius 3 2048^2 11.1 against 9.6.
-const Variant *pick_block(int R, int shape, int64_t ny, int64_t nx) {
-  const bool box = shape == cs::SHAPE_BOX;
-  if (R == 2 || (R == 3 && box) || ny * nx >= (box ? 5000000 : 8000000)) return nullptr;
-  int cnt = 0;
-  const Variant *vs = cs::variants_2d_block(&cnt), *best = nullptr;
-  double best_t = 1e300;
-  for (int i = 0; i < cnt; ++i) {
-    const Variant &v = vs[i];
-    if (v.R != R || v.shape != shape || !fits(&v, ny, nx)) continue;
-    const int64_t wo = v.bx - 2 * R * v.kf, to = v.by - 2 * R * v.kf;
-    const int64_t tiles = (1 + (nx - v.bx + wo - 1) / wo) * (1 + (ny - v.by + to - 1) / to);
-    if (R == 3 && tiles > 256) continue;
-    const double t = block_cost(v, tiles);
-    if (t < best_t) {
-      best_t = t;
-      best = &v;
-    }
-  }
-  return best ? find_variant(2, 11, R, shape, best->kf, best->id) : nullptr;
 }
 
 // The stacked-wave 3-D kernel (k3d_tile.hip) of the least predicted time per step, or null where no
@@ -269,7 +232,6 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
     if (v && nd >= 2 && prec == CS_PREC_FP64 && !fits(v, ny, nx)) v = nullptr;
   } else if (prec == CS_PREC_FP64) {
     if (nd == 2) v = pick_pipe(R, shape, fusion_depth, ny, nx);
-    if (nd == 2 && !v && fusion_depth == 0) v = pick_block(R, shape, ny, nx);
     if (nd == 3 && fusion_depth == 0) v = pick_tile3(R, shape, nz, ny, nx);
     if (v) return v;
     // 1-D: the register-resident kernels (mf 6) at their deepest compiled fusion, else the
@@ -314,6 +276,16 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
   return v;
 }
 
+// Prepares every variant that a sequence may take.
+cs_status prepare_sequence(const cs::Sequence2D &s) {
+  hipError_t e = hipSuccess;
+  s.each_variant([&](const Variant *v) {
+    if (e == hipSuccess) e = v->prepare();
+  });
+  CS_HIP(e);
+  return CS_OK;
+}
+
 cs_status select_variants(cs_plan *p) {
   const int nd = p->ndim;
   const int prec = p->opt.precision;
@@ -332,7 +304,12 @@ cs_status select_variants(cs_plan *p) {
   const bool deep = nd == 2 && p->R == 3 && p->shape == cs::SHAPE_BOX && p->opt.fusion_depth == 0 &&
                     p->opt.tile_variant <= 0 && (prec == CS_PREC_FP16W3 || prec == CS_PREC_BF16X3);
   const Variant *v = nullptr;
-  if (p->opt.tile_variant > 0) {
+  p->by_time = nd == 2 && prec == CS_PREC_FP64 && p->opt.fusion_depth == 0 && p->opt.tile_variant <= 0 &&
+               p->seq[1].init(p->R, p->shape, p->L.n[1], p->L.n[2], true) &&
+               p->seq[0].init(p->R, p->shape, p->L.n[1], p->L.n[2], false);
+  if (p->by_time) {
+    v = p->seq[1].main();
+  } else if (p->opt.tile_variant > 0) {
     v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2],
                   p->L.n[0]);
     if (!v) return CS_ERR_INVALID;
@@ -358,15 +335,18 @@ cs_status select_variants(cs_plan *p) {
   p->vmain = v;
   // single-step launches: the chosen variant itself when it is a single-step one (a variant
   // forced by id must be the one that runs), else the family's first single-step variant
-  p->vone = prec == CS_PREC_FP64 ? single_step(nd, p->R, p->shape, v)
-                                  : v->kf == 1 ? v : find_variant(nd, v->mf, p->R, p->shape, 1, 0, prec, fam);
+  p->vone = p->by_time              ? p->seq[1].one()
+            : prec == CS_PREC_FP64 ? single_step(nd, p->R, p->shape, v)
+            : v->kf == 1           ? v
+                                   : find_variant(nd, v->mf, p->R, p->shape, 1, 0, prec, fam);
   if (!p->vone) return CS_ERR_UNSUPPORTED;
   p->vrem.assign(v->kf, nullptr);
-  for (int r = 1; r < v->kf; ++r)
+  for (int r = 1; r < v->kf && !p->by_time; ++r)
     p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
   for (const Variant *u : {p->vmain, p->vone}) CS_HIP(u->prepare());
   for (const Variant *u : p->vrem)
     if (u) CS_HIP(u->prepare());
+  if (p->by_time) CS_TRY(prepare_sequence(p->seq[1]));
   if (prec != CS_PREC_FP64) {
     std::vector<unsigned char> hb(1 << 20);
     const size_t bytes = nd == 3      ? cs::build_bfrag_split3(prec, p->R, p->shape, p->w.data(), hb.data(), hb.size())
@@ -384,11 +364,11 @@ cs_status select_variants(cs_plan *p) {
   // those whose single steps run on an MFMA kernel (mf 7 and 10: the 2-D 4 x 4 x 4 kernel, mf 9
   // and 12: the 3-D 8 x 8 blocks) appends that kernel's B fragments
   p->frag_off = 0;
-  if (v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10 || v->mf == 11 ||
-      v->mf == 12) {
+  if (p->by_time || v->mf == 1 || v->mf == 2 || v->mf == 3 || v->mf == 7 || v->mf == 9 || v->mf == 10 ||
+      v->mf == 11 || v->mf == 12) {
     std::vector<double> h((p->w.size() + 63) / 64 * 64, 0.0);
     std::copy(p->w.begin(), p->w.end(), h.begin());
-    if ((v->mf == 7 || v->mf == 10 || v->mf == 11) && p->vone->mf == 4) {
+    if ((p->by_time || v->mf == 7 || v->mf == 10 || v->mf == 11) && p->vone->mf == 4) {
       p->frag_off = (int64_t)h.size();
       h.resize(h.size() + (size_t)cs::bfrag_ksteps_2d_f64(4, p->R, p->shape) * 64);
       cs::build_bfrag_2d_f64(4, p->R, p->shape, p->w.data(), h.data() + p->frag_off);
@@ -444,6 +424,14 @@ bool fuses(const cs_plan *p) {
   return p->halo_uniform || (p->opt.precision == CS_PREC_FP64 && (p->vmain->mf == 10 || p->vmain->mf == 11));
 }
 
+// Steps per launch of a run of `steps` steps, as reported: the deepest launch's.
+int32_t executed_depth(const cs_plan *p, int64_t steps) {
+  if (!p->by_time || steps <= 0) return fuses(p) ? p->vmain->kf : 1;
+  int d = 1;
+  p->seq[p->halo_uniform].each(steps, [&](const Variant *v, int64_t) { d = std::max(d, v->kf); });
+  return d;
+}
+
 // Launch sequence for `steps` physical steps.  With uniform halos, fused
 // launches are exact: take the main depth as often as it fits, then the largest
 // compiled depth that fits the rest.  Otherwise every launch is a single step so
@@ -457,6 +445,11 @@ bool fuses(const cs_plan *p) {
 void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *> *seq) {
   seq->clear();
   if (steps <= 0) return;
+  if (p->by_time) {
+    p->seq[p->halo_uniform].each(
+        steps, [&](const Variant *v, int64_t n) { seq->insert(seq->end(), (size_t)n, v); });
+    return;
+  }
   if (!fuses(p) || p->vmain->kf == 1) {
     seq->assign((size_t)steps, p->vone);
     return;
@@ -777,9 +770,17 @@ void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> 
   }
 }
 
+// Predicted us per step of a launch of the register-tile kernel v over `tiles` tiles: about 4.5 us +
+// c (1.2 + a kf) us a launch, c = tiles per CU (at least 1).
+double block_cost(const Variant &v, int64_t tiles) {
+  const bool box = v.shape == cs::SHAPE_BOX;
+  const double a = v.R == 3 ? 3.1 : box ? (v.st == 4 ? 0.55 : 0.93) : (v.st == 4 ? 0.42 : 0.75);
+  const double c = v.R == 3 ? (double)((tiles + 255) / 256) : std::max(1.0, (double)tiles / 256);
+  return (4.5 + c * (1.2 + a * v.kf)) / v.kf;
+}
+
 // The same for the register-tile kernels, for several grids of one stencil that share their launches
-// (sizes: rows, columns): empty when there is no tile that fits them all.  A launch of depth kf takes what
-// pick_block says, with the tiles of all grids (radius 3, one workgroup per CU: whole rounds).
+// (sizes: rows, columns): empty when there is no tile that fits them all.
 cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, int64_t>> &sizes, int64_t steps,
                          std::vector<const Variant *> *seq) {
   seq->clear();
@@ -938,6 +939,7 @@ cs_status cs_plan_upload(cs_plan *p, const double *host_in) {
   p->cur = 0;
   p->steps_done = 0;
   p->halo_uniform = halo_is_zero(&p->L, host_in);
+  if (p->by_time && !p->halo_uniform) CS_TRY(prepare_sequence(p->seq[0]));
   // the scan (5.2 ms for 2048^2, of 11 ms for a whole host-to-host run) serves the FP16 range guard only
   p->amax = p->opt.precision == CS_PREC_FP16X2 || p->opt.precision == CS_PREC_FP16W3 ? abs_max(host_in, n) : 0.0;
   return CS_OK;
@@ -969,7 +971,7 @@ cs_status cs_plan_run(cs_plan *p, int64_t steps, cs_report *rep) {
   if (rep) {
     memset(rep, 0, sizeof(*rep));
     rep->launches = p->launches - l0;
-    rep->fusion_depth = fuses(p) ? p->vmain->kf : 1;
+    rep->fusion_depth = executed_depth(p, steps);
     rep->variant = p->vmain->id;
   }
   return CS_OK;
@@ -1002,7 +1004,7 @@ cs_status cs_plan_time(cs_plan *p, int64_t steps, int32_t warmup, int32_t reps, 
     // a grid without interior cells launches nothing: no rate
     rep->gstencil_per_s = rep->elapsed_ms > 0 && pts > 0 ? pts * (double)steps / (rep->elapsed_ms * 1e-3) / 1e9 : 0.0;
     rep->launches = (p->launches - l0) / reps;
-    rep->fusion_depth = fuses(p) ? p->vmain->kf : 1;
+    rep->fusion_depth = executed_depth(p, steps);
     rep->variant = p->vmain->id;
   }
   return CS_OK;
@@ -1061,7 +1063,7 @@ cs_status cs_run(const cs_layout *layout, const cs_stencil *st, const double *ho
     const double pts = (double)layout->n[0] * (double)layout->n[1] * (double)layout->n[2];
     rep->gstencil_per_s = ms > 0 ? pts * (double)steps / (ms * 1e-3) / 1e9 : 0.0;
     rep->launches = p->launches - l0;
-    rep->fusion_depth = fuses(p) ? p->vmain->kf : 1;
+    rep->fusion_depth = executed_depth(p, steps);
     rep->variant = p->vmain->id;
   }
   if (e0) (void)hipEventDestroy(e0);

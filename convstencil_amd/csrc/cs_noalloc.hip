@@ -13,6 +13,7 @@
 #include <atomic>
 
 #include "cs_host_util.h"
+#include "cs_sequence.h"
 #include "cs_internal.h"
 
 namespace cs {
@@ -22,8 +23,8 @@ cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int t
 
 namespace {
 
-// B fragments of one 2-D FP64 plan: at most 16 k-steps (radius-3 box) x 64 lanes.
-constexpr int kScratchDoubles = 16 * 64;
+// Dense weights (64) and B fragments of one 2-D FP64 plan: at most 16 k-steps (radius-3 box) x 64 lanes.
+constexpr int kScratchDoubles = 64 + 16 * 64;
 constexpr int kMaxDevices = 64;
 
 // Compact fragments: lane l of k-step ks holds value (ks, l >> 4, l & 3) -- the dilated
@@ -90,15 +91,29 @@ extern "C" cs_status cs_run_2d_noalloc(const cs_layout *layout, const cs_stencil
   int dev = 0;
   CS_TRY(check_device(&dev));
   const int shape = classify_2d(R, st->weights);
+  const bool empty = layout->n[1] == 0 || layout->n[2] == 0;
   const cs::Variant *vmain = nullptr, *vone = nullptr, *vrem[32] = {};
-  CS_TRY(cs::pick_fp64_variants(2, R, shape, o.fusion_depth, o.tile_variant, layout->n[1], layout->n[2],
-                                &vmain, &vone, vrem, 32));
+  // a caller without a wish gets a plan's own sequence
+  cs::Sequence2D seq;
+  const bool by_time =
+      o.fusion_depth == 0 && o.tile_variant <= 0 && seq.init(R, shape, layout->n[1], layout->n[2], true);
+  if (by_time) {
+    vmain = seq.main();
+    vone = seq.one();
+  } else {
+    CS_TRY(cs::pick_fp64_variants(2, R, shape, o.fusion_depth, o.tile_variant, layout->n[1], layout->n[2], &vmain,
+                                  &vone, vrem, 32));
+  }
   // the dilated tables (mf 4: B fragments) and the register-streaming, level-pipelined
   // and register-tile kernels (mf 7, 10, 11: dense weights, their single steps on the mf 4 kernel as in a plan):
-  // scratch holds the dense weights first when the main variant is one of those, then the B
-  // fragments when an mf 4 kernel runs
-  const bool dense = vmain->mf == 7 || vmain->mf == 10 || vmain->mf == 11, frags4 = vmain->mf == 4 || vone->mf == 4;
-  if (vmain->mf != 4 && !dense) return CS_ERR_UNSUPPORTED;
+  // scratch holds the dense weights first when one of those runs, then the B
+  // fragments when an mf 4 kernel does
+  bool dense = vmain->mf == 7 || vmain->mf == 10 || vmain->mf == 11, frags4 = vmain->mf == 4 || vone->mf == 4;
+  if (by_time) {
+    dense = frags4 = false;
+    if (steps > 0) seq.each(steps, [&](const cs::Variant *v, int64_t) { (v->mf == 4 ? frags4 : dense) = true; });
+  }
+  if (!by_time && vmain->mf != 4 && !dense) return CS_ERR_UNSUPPORTED;
   const int D = 2 * R + 1;
   const int nks = frags4 ? cs::bfrag_ksteps_2d_f64(4, R, vmain->shape) : 0;
   const int64_t off4 = dense ? 64 : 0;  // doubles before the B fragments
@@ -132,10 +147,9 @@ extern "C" cs_status cs_run_2d_noalloc(const cs_layout *layout, const cs_stencil
   if (frags4)
     hipLaunchKernelGGL(cs::expand_frags, dim3((nks * 64 + 255) / 256), dim3(256), 0, s, cf, nks, 0, frags + off4);
   CS_HIP(hipGetLastError());
-  for (const cs::Variant *u : {vmain, vone}) CS_HIP(u->prepare());
   // the reference's ping-pong: fused launches are exact when both buffers carry the same
   // halo (the caller's contract); fusion_depth 1 gives the alternating-halo single steps
-  if (layout->n[1] == 0 || layout->n[2] == 0) {
+  if (empty) {
     if (final_buffer) *final_buffer = (int32_t)(steps & 1);
     return CS_OK;
   }
@@ -148,22 +162,32 @@ extern "C" cs_status cs_run_2d_noalloc(const cs_layout *layout, const cs_stencil
   g.tiles[0] = 1;
   double *b[2] = {buf0, buf1};
   int cur = 0;
-  int64_t left = steps;
-  while (left > 0) {
-    const cs::Variant *v = vone;
-    if (left >= vmain->kf) {
-      v = vmain;
-    } else {
-      for (int r = 1; r < vmain->kf; ++r)
-        if (vrem[r] && vrem[r]->kf <= left && vrem[r]->kf > v->kf) v = vrem[r];
-    }
-    if (v != vmain && v != vone) CS_HIP(v->prepare());
+  hipError_t e = hipSuccess;
+  auto launches = [&](const cs::Variant *v, int64_t n) {
+    if (e == hipSuccess) e = v->prepare();
     g.tiles[1] = (layout->n[1] + v->by - 1) / v->by;
     g.tiles[2] = (layout->n[2] + v->bx - 1) / v->bx;
-    CS_HIP(v->launch(b[cur], b[cur ^ 1], v->mf == 4 ? frags + off4 : frags, g, s));
-    cur ^= 1;
-    left -= v->kf;
+    for (int64_t i = 0; i < n && e == hipSuccess; ++i) {
+      e = v->launch(b[cur], b[cur ^ 1], v->mf == 4 ? frags + off4 : frags, g, s);
+      cur ^= 1;
+    }
+  };
+  if (by_time) {
+    if (steps > 0) seq.each(steps, launches);
+  } else {
+    for (int64_t left = steps; left > 0 && e == hipSuccess;) {
+      const cs::Variant *v = vone;
+      if (left >= vmain->kf) {
+        v = vmain;
+      } else {
+        for (int r = 1; r < vmain->kf; ++r)
+          if (vrem[r] && vrem[r]->kf <= left && vrem[r]->kf > v->kf) v = vrem[r];
+      }
+      launches(v, 1);
+      left -= v->kf;
+    }
   }
+  CS_HIP(e);
   if (final_buffer) *final_buffer = cur;
   return CS_OK;
 }

@@ -38,6 +38,11 @@ int32_t cs_debug_variant_count(int32_t ndim);
  * variants: the z-chunk length), LDS storage column of tile column 0 (2-D 4x4x4 variants, else 0).
  * Returns 0, or -1 if i is out of range.  name receives the variant's name. */
 int32_t cs_debug_variant_info(int32_t ndim, int32_t i, int64_t *info, char *name, int32_t len);
+/* The launches that a default 2-D FP64 plan makes for `steps` steps (cs_sequence.cpp): entry i is
+ * counts[i] launches of variant ids[i], in order; zero_halo = 0: an uploaded halo.  Returns the number of
+ * entries, -1 if cap is too small, or 0 where the plan takes another rule. */
+int32_t cs_debug_sequence_2d(int32_t radius, int32_t shape, int64_t ny, int64_t nx, int32_t zero_halo, int64_t steps,
+                             int32_t *ids, int64_t *counts, int32_t cap);
 /* k-step table of the 16x16x4 kernels (mf = 16) or the flattened 4x4x4 table of the 1-D kernels'
  * layout (mf = 4): dy[], c0[], live[] (cap entries each); returns the table length, or -1. */
 int32_t cs_debug_ktable(int32_t mf, int32_t radius, int32_t shape, int32_t *dy, int32_t *c0, int32_t *live,
