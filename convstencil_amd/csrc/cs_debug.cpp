@@ -63,6 +63,21 @@ int32_t cs_debug_sequence_2d(int32_t radius, int32_t shape, int64_t ny, int64_t 
   return n > cap ? -1 : n;
 }
 
+int32_t cs_debug_sequence_3d(int32_t radius, int32_t shape, int64_t nz, int64_t ny, int64_t nx, int64_t steps,
+                             int32_t *ids, int64_t *counts, int32_t cap) {
+  cs::Sequence3D q;
+  if (steps < 2 || !ids || !counts || !q.init(radius, shape, nz, ny, nx)) return 0;
+  int n = 0;
+  q.each(steps, [&](const cs::Variant *v, int64_t count) {
+    if (n < cap) {
+      ids[n] = v->id;
+      counts[n] = count;
+    }
+    ++n;
+  });
+  return n > cap ? -1 : n;
+}
+
 int32_t cs_debug_ktable(int32_t mf, int32_t radius, int32_t shape, int32_t *dy, int32_t *c0, int32_t *live,
                         int32_t cap) {
   const cs::KTable t = mf == 16 ? cs::make_ktable(radius, shape) : cs::make_ftable(radius, shape);

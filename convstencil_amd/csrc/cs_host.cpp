@@ -49,6 +49,8 @@ struct cs_plan {
   // 2-D FP64 plans that choose for themselves: the sequences for a zero halo [1] and another one [0]
   bool by_time = false;
   cs::Sequence2D seq[2];
+  bool by_time3 = false;  // 3-D ones on the stacked-wave kernels (zero halos)
+  cs::Sequence3D seq3;
   std::map<std::pair<int64_t, int>, hipGraphExec_t> graphs;
   int64_t launches = 0;
   int tuned = 0;  // 0 defaults or a forced variant, 1 cached autotuner choice, 2 timed now
@@ -199,28 +201,10 @@ const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t
   return find_variant(2, 10, R, shape, depth, 0);
 }
 
-// The stacked-wave 3-D kernel (k3d_tile.hip) of the least predicted time per step, or null where no
-// tile fits (fewer than 64 columns or 24 rows): the other families lose on every grid measured
-// that one fits, from 2% (box 40 x 500 x 500) to 4.6 times (box 64^3 22 -> 4.9 us).
-const Variant *pick_tile3(int R, int shape, int64_t nz, int64_t ny, int64_t nx) {
-  int cnt = 0;
-  const Variant *vs = cs::variants_3d_tile(&cnt), *best = nullptr;
-  double best_t = 1e300;
-  for (int i = 0; i < cnt; ++i) {
-    if (vs[i].R != R || vs[i].shape != shape || nz < 1 || !fits(&vs[i], ny, nx)) continue;
-    const double t = cs::tile3_cost(vs[i], nz, ny, nx);
-    if (t < best_t) {
-      best_t = t;
-      best = &vs[i];
-    }
-  }
-  return best ? find_variant(3, 12, R, shape, best->kf, best->id) : nullptr;
-}
-
-// The main variant of a plan: a forced id, else the preferred family's default depth (nz x ny x nx
-// = the interior of one grid, 0 when no single grid decides).
+// The main variant of a plan: a forced id, else the preferred family's default depth (ny x nx = the
+// interior of one grid, 0 when no single grid decides).
 const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, int tile_variant, int64_t ny = 0,
-                         int64_t nx = 0, int64_t nz = 0) {
+                         int64_t nx = 0) {
   const int64_t cells = nd == 2 ? ny * nx : 0;
   const int mf = prec != CS_PREC_FP64 ? prec : 4;
   const Variant *v = nullptr;
@@ -232,7 +216,6 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
     if (v && nd >= 2 && prec == CS_PREC_FP64 && !fits(v, ny, nx)) v = nullptr;
   } else if (prec == CS_PREC_FP64) {
     if (nd == 2) v = pick_pipe(R, shape, fusion_depth, ny, nx);
-    if (nd == 3 && fusion_depth == 0) v = pick_tile3(R, shape, nz, ny, nx);
     if (v) return v;
     // 1-D: the register-resident kernels (mf 6) at their deepest compiled fusion, else the
     // 4 x 4 x 4 blocks; 2-D: the register-streaming kernels (mf 7), else the dilated 8 x 8
@@ -277,7 +260,8 @@ const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, i
 }
 
 // Prepares every variant that a sequence may take.
-cs_status prepare_sequence(const cs::Sequence2D &s) {
+template <class S>
+cs_status prepare_sequence(const S &s) {
   hipError_t e = hipSuccess;
   s.each_variant([&](const Variant *v) {
     if (e == hipSuccess) e = v->prepare();
@@ -307,14 +291,19 @@ cs_status select_variants(cs_plan *p) {
   p->by_time = nd == 2 && prec == CS_PREC_FP64 && p->opt.fusion_depth == 0 && p->opt.tile_variant <= 0 &&
                p->seq[1].init(p->R, p->shape, p->L.n[1], p->L.n[2], true) &&
                p->seq[0].init(p->R, p->shape, p->L.n[1], p->L.n[2], false);
+  // where a tile fits (64 columns, 24 rows) the other 3-D families lose on every grid measured, from 2% (box
+  // 40 x 500 x 500) to 4.6 times (box 64^3 22 -> 4.9 us a step)
+  p->by_time3 = nd == 3 && prec == CS_PREC_FP64 && p->opt.fusion_depth == 0 && p->opt.tile_variant <= 0 &&
+                p->seq3.init(p->R, p->shape, p->L.n[0], p->L.n[1], p->L.n[2]);
   if (p->by_time) {
     v = p->seq[1].main();
+  } else if (p->by_time3) {
+    v = p->seq3.main();
   } else if (p->opt.tile_variant > 0) {
-    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2],
-                  p->L.n[0]);
+    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, p->opt.tile_variant, p->L.n[1], p->L.n[2]);
     if (!v) return CS_ERR_INVALID;
   } else if (prec == CS_PREC_FP64) {
-    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, 0, p->L.n[1], p->L.n[2], p->L.n[0]);
+    v = pick_main(nd, p->R, p->shape, prec, p->opt.fusion_depth, 0, p->L.n[1], p->L.n[2]);
   } else {
     const int tries[3][2] = {{p->shape, 2}, {cs::SHAPE_BOX, 2}, {cs::SHAPE_BOX, 0}};
     for (const auto &tr : tries) {
@@ -341,12 +330,13 @@ cs_status select_variants(cs_plan *p) {
                                    : find_variant(nd, v->mf, p->R, p->shape, 1, 0, prec, fam);
   if (!p->vone) return CS_ERR_UNSUPPORTED;
   p->vrem.assign(v->kf, nullptr);
-  for (int r = 1; r < v->kf && !p->by_time; ++r)
+  for (int r = 1; r < v->kf && !p->by_time && !p->by_time3; ++r)
     p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
   for (const Variant *u : {p->vmain, p->vone}) CS_HIP(u->prepare());
   for (const Variant *u : p->vrem)
     if (u) CS_HIP(u->prepare());
   if (p->by_time) CS_TRY(prepare_sequence(p->seq[1]));
+  if (p->by_time3) CS_TRY(prepare_sequence(p->seq3));
   if (prec != CS_PREC_FP64) {
     std::vector<unsigned char> hb(1 << 20);
     const size_t bytes = nd == 3      ? cs::build_bfrag_split3(prec, p->R, p->shape, p->w.data(), hb.data(), hb.size())
@@ -426,9 +416,13 @@ bool fuses(const cs_plan *p) {
 
 // Steps per launch of a run of `steps` steps, as reported: the deepest launch's.
 int32_t executed_depth(const cs_plan *p, int64_t steps) {
-  if (!p->by_time || steps <= 0) return fuses(p) ? p->vmain->kf : 1;
+  if ((!p->by_time && !(p->by_time3 && p->halo_uniform)) || steps <= 0) return fuses(p) ? p->vmain->kf : 1;
   int d = 1;
-  p->seq[p->halo_uniform].each(steps, [&](const Variant *v, int64_t) { d = std::max(d, v->kf); });
+  auto deepest = [&](const Variant *v, int64_t) { d = std::max(d, v->kf); };
+  if (p->by_time)
+    p->seq[p->halo_uniform].each(steps, deepest);
+  else if (steps > 1)
+    p->seq3.each(steps, deepest);
   return d;
 }
 
@@ -448,6 +442,10 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
   if (p->by_time) {
     p->seq[p->halo_uniform].each(
         steps, [&](const Variant *v, int64_t n) { seq->insert(seq->end(), (size_t)n, v); });
+    return;
+  }
+  if (p->by_time3 && p->halo_uniform && steps > 1) {
+    p->seq3.each(steps, [&](const Variant *v, int64_t n) { seq->insert(seq->end(), (size_t)n, v); });
     return;
   }
   if (!fuses(p) || p->vmain->kf == 1) {

@@ -1,4 +1,4 @@
-// cs_sequence.cpp -- which kernels run a number of steps of a 2-D FP64 grid.
+// cs_sequence.cpp -- which kernels run a number of steps of a 2-D or 3-D FP64 grid.
 //
 // Four families compete (radius-1 box and star, radius-3 star and box): MFMA tables (mf 4),
 // register-streaming strips (mf 7), level-pipelined strips (mf 10) and register tiles (mf 11), each
@@ -256,6 +256,72 @@ Sequence2D::Cut Sequence2D::even_cut(int64_t steps) const {
     }
   }
   return best;
+}
+
+bool Sequence3D::init(int R, int shape, int64_t nz, int64_t ny, int64_t nx) {
+  std::fill(depth_, depth_ + kDepths + 1, nullptr);
+  std::fill(us_, us_ + kDepths + 1, kInf);
+  bulk_ = nullptr;
+  int n = 0;
+  const Variant *vs = variants_3d_tile(&n);
+  for (int i = 0; i < n; ++i) {
+    const Variant &v = vs[i];
+    if (v.R != R || v.shape != shape || v.kf < 2 || v.kf > kDepths || nz < 1 || nx < v.bx || ny < v.by) continue;
+    const double us = tile3_cost(v, nz, ny, nx) * v.kf;
+    if (us < us_[v.kf]) {
+      us_[v.kf] = us;
+      depth_[v.kf] = &v;
+    }
+  }
+  for (int k = 2; k <= kDepths; ++k)
+    if (depth_[k] && (!bulk_ || us_[k] / k < us_[bulk_->kf] / bulk_->kf)) bulk_ = depth_[k];
+  // the other depths on the same tile unless another one is predicted to be 15% faster (star 10 x 2000 x 66, 5
+  // steps, 36.3 us on one tile, 40.0 on two)
+  for (int i = 0; bulk_ && i < n; ++i) {
+    const Variant &v = vs[i];
+    if (v.R != R || v.shape != shape || v.by != bulk_->by || v.nw != bulk_->nw || v.kf < 2 || v.kf > kDepths) continue;
+    const double us = tile3_cost(v, nz, ny, nx) * v.kf;
+    if (us <= 1.15 * us_[v.kf]) {
+      us_[v.kf] = us;
+      depth_[v.kf] = &v;
+    }
+  }
+  return depth_[2] && depth_[3];  // together they make every number from 2 up
+}
+
+double Sequence3D::cost(const int64_t *count) const {
+  double us = -4.0;  // every change of variant counts as in two dimensions (Sequence2D)
+  for (int k = 2; k <= kDepths; ++k)
+    if (count[k] > 0) us += (double)count[k] * us_[k] + 4.0;
+  return us;
+}
+
+// As few launches as the main depth allows, cut evenly, unless another mix is predicted to be 5% faster.  An
+// odd number of steps never leaves one for the single-step kernel: radius-1 star 30 x 24 x 1000, 3 steps as
+// 2 + 1 72 us, as one launch 18.
+void Sequence3D::choose(int64_t steps, int64_t *count) const {
+  const int kf = bulk_->kf;
+  double least = kInf;
+  const int64_t launches = ceil_div(steps, kf), d = steps / launches, deeper = steps % launches;
+  if (d >= 2) {
+    count[d] = launches - deeper;
+    if (deeper > 0) count[d + 1] = deeper;
+    least = 0.95 * cost(count);
+  }
+  const int64_t n = steps > kSteps ? ceil_div(steps - kSteps, kf) : 0;
+  const int rest = (int)(steps - n * kf);
+  for (int four = 0; 4 * four <= rest && (four == 0 || depth_[4]); ++four)
+    for (int three = 0; 4 * four + 3 * three <= rest; ++three) {
+      const int left = rest - 4 * four - 3 * three;
+      if (left % 2) continue;
+      int64_t c[kDepths + 1] = {0, 0, left / 2, three, four};
+      c[kf] += n;
+      const double us = cost(c);
+      if (us < least) {
+        least = us;
+        std::copy(c, c + kDepths + 1, count);
+      }
+    }
 }
 
 }  // namespace cs

@@ -1,4 +1,4 @@
-// cs_sequence.h -- launch sequences of least predicted time for 2-D FP64 grids (cs_sequence.cpp).
+// cs_sequence.h -- launch sequences of least predicted time for 2-D and 3-D FP64 grids (cs_sequence.cpp).
 #pragma once
 #include "cs_internal.h"
 
@@ -128,6 +128,37 @@ class Sequence2D {
   // a launch of even depth puts it into the other one.
   double us_[2][kSteps + 1];
   signed char pick_[2][kSteps + 1];
+};
+
+// The same for the stacked-wave 3-D kernels (k3d_tile.hip; zero halo): depths 2, 3 and, where compiled, 4,
+// each on the tile of its least predicted time.  One step has no launch of theirs.
+class Sequence3D {
+ public:
+  // False where no tile fits the grid.
+  bool init(int R, int shape, int64_t nz, int64_t ny, int64_t nx);
+  const Variant *main() const { return bulk_; }
+  // f(variant, count) for consecutive launches of steps >= 2 steps.
+  template <class F>
+  void each(int64_t steps, F f) const {
+    int64_t count[kDepths + 1] = {};
+    choose(steps, count);
+    for (int k = kDepths; k >= 2; --k)
+      if (count[k] > 0) f(depth_[k], count[k]);
+  }
+  template <class F>
+  void each_variant(F f) const {
+    for (int k = 2; k <= kDepths; ++k)
+      if (depth_[k]) f(depth_[k]);
+  }
+
+ private:
+  static constexpr int kSteps = 24, kDepths = 4;
+  // Launches per depth, and their time with the changes of variant.
+  void choose(int64_t steps, int64_t *count) const;
+  double cost(const int64_t *count) const;
+  const Variant *depth_[kDepths + 1] = {};
+  double us_[kDepths + 1];
+  const Variant *bulk_ = nullptr;
 };
 
 }  // namespace cs

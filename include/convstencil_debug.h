@@ -43,6 +43,9 @@ int32_t cs_debug_variant_info(int32_t ndim, int32_t i, int64_t *info, char *name
  * entries, -1 if cap is too small, or 0 where the plan takes another rule. */
 int32_t cs_debug_sequence_2d(int32_t radius, int32_t shape, int64_t ny, int64_t nx, int32_t zero_halo, int64_t steps,
                              int32_t *ids, int64_t *counts, int32_t cap);
+/* The same for 3-D plans with a zero halo on the stacked-wave kernels (steps >= 2). */
+int32_t cs_debug_sequence_3d(int32_t radius, int32_t shape, int64_t nz, int64_t ny, int64_t nx, int64_t steps,
+                             int32_t *ids, int64_t *counts, int32_t cap);
 /* k-step table of the 16x16x4 kernels (mf = 16) or the flattened 4x4x4 table of the 1-D kernels'
  * layout (mf = 4): dy[], c0[], live[] (cap entries each); returns the table length, or -1. */
 int32_t cs_debug_ktable(int32_t mf, int32_t radius, int32_t shape, int32_t *dy, int32_t *c0, int32_t *live,

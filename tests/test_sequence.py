@@ -101,3 +101,26 @@ def test_the_faster_family(R, shape, ny, nx, zero, steps, family):
 def test_no_shallow_tiles(ny, nx):
     # radius-3 star, 48 steps: tiles so shallow that each CU has one, 948-1017 us; strips 459-473
     assert all(v["kf"] >= 4 for v, _ in _sequence(3, STAR, ny, nx, 1, 48))
+
+
+@pytest.mark.parametrize("shape", [BOX, STAR])
+def test_3d_steps(shape):
+    # every number of steps from 2 up is made of launches of 2 to 4: none is left for the single-step
+    # kernel (star 30 x 24 x 1000, 3 steps: 2 + 1 72 us, the strips before them 32)
+    LIB.cs_debug_sequence_3d.argtypes = [ctypes.c_int32, ctypes.c_int32] + [ctypes.c_int64] * 4 + [
+        ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64), ctypes.c_int32]
+    depth = {}
+    for i in range(LIB.cs_debug_variant_count(13)):
+        info = (ctypes.c_int64 * 12)()
+        LIB.cs_debug_variant_info(13, i, info, None, 0)
+        depth[int(info[0])] = (int(info[3]), int(info[4]), int(info[5]), int(info[6]))
+    ids, counts = (ctypes.c_int32 * 8)(), (ctypes.c_int64 * 8)()
+    for n in ([1, 24, 64], [30, 24, 1000], [17, 90, 130], [100, 100, 100], [512, 512, 512], [3, 3000, 3000]):
+        for steps in list(range(2, 40)) + [1000, 100001]:
+            k = LIB.cs_debug_sequence_3d(1, shape, *n, steps, ids, counts, 8)
+            assert k > 0
+            got = [(depth[ids[i]], counts[i]) for i in range(k)]
+            assert sum(v[1] * c for v, c in got) == steps
+            assert all(v[0] == shape and v[2] <= n[1] and v[3] <= n[2] and c > 0 for v, c in got)
+    assert LIB.cs_debug_sequence_3d(1, shape, 10, 23, 64, 4, ids, counts, 8) == 0
+    assert LIB.cs_debug_sequence_3d(2, shape, 100, 100, 100, 4, ids, counts, 8) == 0
