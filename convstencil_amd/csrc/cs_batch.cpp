@@ -1,8 +1,8 @@
 // cs_batch.cpp -- host side of the batched workload (cs_batch_* in convstencil.h).
 //
 // FP64 batches whose grids all carry a uniform halo run on the register-tile 2-D kernels
-// (k2d_block.hip), grids too small for a tile on the register-streaming ones
-// (k2d_reg.hip): launch j of the run advances every grid whose launch sequence
+// (k2d_block.hip), stencil classes that are faster without them and grids too small for a tile on the
+// register-streaming ones (k2d_reg.hip): launch j of the run advances every grid whose launch sequence
 // has a j-th launch, all grids of one kernel variant in one multi-grid launch (the kernel
 // boundary orders the steps; no device-wide barrier).  Every other batch runs the
 // persistent kernel: `steps` time steps of every grid become step blocks of work items
@@ -86,7 +86,7 @@ struct cs_batch {
 namespace cs {
 void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> *seq);
 cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, int64_t>> &sizes, int64_t steps,
-                         std::vector<const Variant *> *seq);
+                         std::vector<const Variant *> *seq, double *us);
 }
 
 namespace {
@@ -200,16 +200,43 @@ void reg_items(const cs_batch *b, int g, const cs::Variant *v, int64_t rows, std
   }
 }
 
-// A stencil class of at most this many cells takes tiles: a launch of the streaming kernels lasts as long as
-// its chains of rows, a tile's overlap costs FMAs.  Measured, us per step, streaming / tiles: 16 box
-// grids of 4.8 M cells 11.3 / 5.8, 8 star grids of 2.9 M cells (two of them too narrow for a tile) 15.9 /
-// 13.3; 256 grids of 118 M cells 143 / 259.
-constexpr int64_t kTileCells = 8000000;
-
 int64_t cells(const std::vector<std::pair<int64_t, int64_t>> &sizes) {
   int64_t n = 0;
   for (const auto &s : sizes) n += s.first * s.second;
   return n;
+}
+
+// Predicted us of `steps` steps of a stencil class on the streaming kernels: a launch lasts as long as its chains
+// of rows, or moves and computes the class's cells.  Measured, us a step of 60, mixed sides up to 2048
+// cells: radius-3 star 1 M cells and less 7.7, 2.6 M 8.3, 4.7 M 11.9, 5.5 M 14.8, 7.9 M 18.7, 10.9 M 22.9;
+// radius-1 box 5 M 7.9, 10 M 12.5, 30 M 30, 113 M 92.  Launches of the family's depths, in such steps: radius 1
+// depth 8 8, 4 6, 2 4.5, 1 5.5; radius 3 depth 4 4, 3 2.8, 2 3.8, 1 1.5.
+double stream_us(int R, int64_t steps, int64_t cells) {
+  struct Depth {
+    int kf;
+    double steps;
+  };
+  static const Depth depths[2][4] = {{{8, 8.0}, {4, 6.0}, {2, 4.5}, {1, 5.5}}, {{4, 4.0}, {3, 2.8}, {2, 3.8}, {1, 1.5}}};
+  const double mc = 1e-6 * (double)cells, step = R == 1 ? std::max(8.0, 0.9 * mc) : std::max(7.7, 3.6 + 1.9 * mc);
+  double n = 0.0;
+  for (const Depth &d : depths[R == 1 ? 0 : 1]) {
+    n += d.steps * (double)(steps / d.kf);
+    steps %= d.kf;
+  }
+  return step * n;
+}
+
+// A stencil class's launches on tiles (`seq`), left empty where the streaming kernels are predicted to be faster
+// (uneven grids' tiles take up to 5% more than the prediction) or a grid is smaller than the tiles.
+// Measured, us of 60 steps, tiles / strips: radius-3 star 1.6 M cells 360 / 471, 2.6 M 512 / 496, 3.8 M 635 /
+// 698, 4.7 M 881 / 715, 5.5 M 999 / 888, 10.9 M 1781 / 1371; radius-1 box 5 M 319 / 475, 10 M 563 / 748, 30 M
+// 1576 / 1794, 113 M (256 grids) 5256 / 5497.
+cs_status class_tiles(int R, int shape, const std::vector<std::pair<int64_t, int64_t>> &sizes, int64_t steps,
+                      std::vector<const cs::Variant *> *seq) {
+  double us = 0.0;
+  CS_TRY(cs::block_sequence(R, shape, sizes, steps, seq, &us));
+  if (1.05 * us >= stream_us(R, steps, cells(sizes))) seq->clear();
+  return CS_OK;
 }
 
 // The register path's launches for `steps` steps: launch j groups, per variant, every grid
@@ -236,16 +263,30 @@ cs_status build_rseq(cs_batch *b, int64_t steps, RegSeq *s) {
     sizes[k].emplace_back(L.n[1], L.n[2]);
   }
   std::vector<std::vector<const cs::Variant *>> tiles(classes.size());
-  for (size_t k = 0; k < classes.size(); ++k)
-    if (std::get<2>(classes[k]) && cells(sizes[k]) <= kTileCells)
-      CS_TRY(cs::block_sequence(std::get<0>(classes[k]), std::get<1>(classes[k]), sizes[k], steps, &tiles[k]));
-  // streamed classes: 64-row chunks, shorter ones (down to 16 rows) where those make fewer waves than
-  // the chip has SIMDs, since a launch then lasts as long as one chunk
+  std::vector<int> launch = chain;  // per grid: the class whose launches and stream it shares
+  for (size_t k = 0; k < classes.size(); ++k) {
+    if (!std::get<2>(classes[k])) continue;
+    CS_TRY(class_tiles(std::get<0>(classes[k]), std::get<1>(classes[k]), sizes[k], steps, &tiles[k]));
+    for (const cs::Variant *v : tiles[k]) CS_HIP(v->prepare());
+    if (!tiles[k].empty()) continue;
+    // streamed: in one launch with the narrow grids of the stencil (of one step, 54 us as two launches on two
+    // streams 75)
+    const Class narrow(std::get<0>(classes[k]), std::get<1>(classes[k]), false);
+    for (size_t m = 0; m < classes.size(); ++m)
+      if (classes[m] == narrow) std::replace(launch.begin(), launch.end(), (int)k, (int)m);
+  }
+  // streamed classes: 64-row chunks, shorter ones where those make fewer waves than the chip has SIMDs (radius
+  // 1, down to 16 rows) or than fill them (radius 3: 64, 32 and 16 rows 642, 496, 739 us at 2.6 M cells, 961,
+  // 888, 1121 at 5.5 M, 1391, 1371, 1735 at 10.9 M; 16 rows pay for a few narrow grids, 769 -> 454), since a
+  // launch then lasts as long as one chunk
   std::vector<int64_t> rows(classes.size());
   for (size_t k = 0; k < classes.size(); ++k) {
     int64_t waves = 0;
     for (const auto &n : sizes[k]) waves += (n.second + 127) / 128 * ((n.first + 63) / 64);
-    rows[k] = std::min<int64_t>(64, std::max<int64_t>(16, 64 * waves / 1024));
+    rows[k] = std::get<0>(classes[k]) == 1 ? std::min<int64_t>(64, std::max<int64_t>(16, 64 * waves / 1024))
+              : waves < 200                ? 16
+              : waves < 1000               ? 32
+                                           : 64;
   }
   size_t nj = 0;
   for (int g = 0; g < b->count; ++g) {
@@ -269,7 +310,7 @@ cs_status build_rseq(cs_batch *b, int64_t steps, RegSeq *s) {
         reg_items(b, g, v, rows[(size_t)chain[(size_t)g]], &it);
         c = cache.emplace(key, it).first;
       }
-      std::vector<cs::RegItem> &dst = groups[std::make_pair(v, chain[(size_t)g])];
+      std::vector<cs::RegItem> &dst = groups[std::make_pair(v, launch[(size_t)g])];
       dst.insert(dst.end(), c->second.begin(), c->second.end());
     }
     for (auto &kv : groups) {
@@ -706,6 +747,15 @@ cs_status cs_batch_describe(cs_batch *b, char *buf, int32_t len) {
            reg_path(b) ? "register-streaming" : "persistent", (long long)tiles, b->max_wg,
            cs::batch_lds_bytes(b->prec));
   return CS_OK;
+}
+
+int32_t cs_debug_batch_tiles(int32_t radius, int32_t shape, int32_t n, const int64_t *rows, const int64_t *cols,
+                             int64_t steps) {
+  std::vector<std::pair<int64_t, int64_t>> sizes;
+  for (int32_t i = 0; i < n; ++i) sizes.emplace_back(rows[i], cols[i]);
+  std::vector<const cs::Variant *> seq;
+  if (class_tiles(radius, shape, sizes, steps, &seq) != CS_OK) return -1;
+  return (int32_t)seq.size();
 }
 
 int32_t cs_debug_batch_latch(const uint32_t *flags, int32_t n, int32_t *status) {

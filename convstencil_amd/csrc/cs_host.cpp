@@ -768,19 +768,11 @@ void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> 
   }
 }
 
-// Predicted us per step of a launch of the register-tile kernel v over `tiles` tiles: about 4.5 us +
-// c (1.2 + a kf) us a launch, c = tiles per CU (at least 1).
-double block_cost(const Variant &v, int64_t tiles) {
-  const bool box = v.shape == cs::SHAPE_BOX;
-  const double a = v.R == 3 ? 3.1 : box ? (v.st == 4 ? 0.55 : 0.93) : (v.st == 4 ? 0.42 : 0.75);
-  const double c = v.R == 3 ? (double)((tiles + 255) / 256) : std::max(1.0, (double)tiles / 256);
-  return (4.5 + c * (1.2 + a * v.kf)) / v.kf;
-}
-
 // The same for the register-tile kernels, for several grids of one stencil that share their launches
-// (sizes: rows, columns): empty when there is no tile that fits them all.
+// (sizes: rows, columns), cut evenly, and its predicted time (*us): empty when there is no tile that
+// fits them all.  The caller prepares them.
 cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, int64_t>> &sizes, int64_t steps,
-                         std::vector<const Variant *> *seq) {
+                         std::vector<const Variant *> *seq, double *us) {
   seq->clear();
   int cnt = 0;
   const Variant *vs = variants_2d_block(&cnt), *best = nullptr;
@@ -789,26 +781,31 @@ cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, 
     const Variant &v = vs[i];
     if (v.R != R || v.shape != shape || v.kf > steps) continue;
     const int64_t wo = v.bx - 2 * R * v.kf, to = v.by - 2 * R * v.kf;
-    int64_t tiles = 0;
+    int64_t tiles = 0, edge = 0;
+    double cells = 0.0;
     bool ok = !sizes.empty();
     for (const auto &n : sizes) {
       ok = ok && fits(&v, n.first, n.second);
-      if (ok) tiles += (1 + (n.second - v.bx + wo - 1) / wo) * (1 + (n.first - v.by + to - 1) / to);
+      if (!ok) break;
+      const int64_t tx = 1 + (n.second - v.bx + wo - 1) / wo, ty = 1 + (n.first - v.by + to - 1) / to;
+      tiles += tx * ty;
+      edge += std::min<int64_t>(tx, 2) * ty;
+      cells += (double)n.first * (double)n.second;
     }
     if (!ok) continue;
-    const double t = block_cost(v, tiles);
+    const double t = tiles_us_2d(v, tiles, edge, cells) / v.kf;
     if (t < best_t) {
       best_t = t;
       best = &v;
     }
   }
   if (!best) return CS_OK;
+  *us = best_t * (double)steps;
   const int64_t n = (steps + best->kf - 1) / best->kf;
   for (int64_t i = 0; i < n; ++i) {
     const int64_t d = steps / n + (i < steps % n);
     const Variant *u = find_variant(2, 11, R, shape, (int)d, 0, CS_PREC_FP64, best->st);
     if (!u) return CS_ERR_UNSUPPORTED;
-    CS_HIP(u->prepare());
     seq->push_back(u);
   }
   return CS_OK;

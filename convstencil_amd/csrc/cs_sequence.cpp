@@ -75,19 +75,27 @@ const TileFit kTile[2][5] = {
      {3, SHAPE_STAR, 8, 8.0, 5.0, 0.101, 7.51, 0.496, 2.56}},
 };
 
+double tile_us(const Variant &v, const TileFit &f, int64_t tiles, int64_t edge, double cells) {
+  const double cu = (double)ceil_div(tiles, (int64_t)kCus), mb = 8e-6 * ((double)tiles * v.by * v.bx + cells);
+  return f.a + f.each * cu + f.mb * mb + f.edge * (double)edge / kCus + v.kf * (f.lat + f.issue * cu);
+}
+
 double tile_us(const Variant &v, const TileFit &f, int64_t ny, int64_t nx) {
   const int64_t tx = 1 + ceil_div(nx - v.bx, v.bx - 2 * v.R * v.kf), ty = 1 + ceil_div(ny - v.by, v.by - 2 * v.R * v.kf);
-  const int64_t tiles = tx * ty, cu = ceil_div(tiles, (int64_t)kCus);
-  const double mb = 8e-6 * ((double)tiles * v.by * v.bx + (double)ny * (double)nx);
-  double t = f.a + f.each * (double)cu + f.mb * mb + f.edge * (double)(std::min<int64_t>(tx, 2) * ty) / kCus +
-             v.kf * (f.lat + f.issue * (double)cu);
+  double t = tile_us(v, f, tx * ty, std::min<int64_t>(tx, 2) * ty, (double)ny * (double)nx);
   // one or two steps with several tiles on a CU, and on narrow grids, where every tile looks at the halo:
   // 7219 x 135, 2 steps, 14.0 us against 11.0 in strips
   if (v.kf < 3 && tx <= 2 && ty > 16)
     t += 6.0;
-  else if (v.kf < 3 && cu > 1)
+  else if (v.kf < 3 && tx * ty > (int64_t)kCus)
     t += 4.0;
   return t;
+}
+
+const TileFit *tile_fit(const Variant &v, bool zero) {
+  for (const TileFit &f : kTile[zero ? 0 : 1])
+    if (f.R == v.R && f.shape == v.shape && f.rows == v.st) return &f;
+  return nullptr;
 }
 
 // Register-streaming strips (zero halos): the longest edge or inner chunk or the sum of all rows over 1024
@@ -159,9 +167,8 @@ double launch_us_2d(const Variant &v, int64_t ny, int64_t nx, bool zero) {
   if (v.mf == 11) {
     // 12 M cells: the largest grid fitted; the pipelines are twice as fast there
     if (ny < v.by || nx < v.bx || (double)ny * (double)nx > 12e6) return kInf;
-    for (const TileFit &f : kTile[zero ? 0 : 1])
-      if (f.R == v.R && f.shape == v.shape && f.rows == v.st) return tile_us(v, f, ny, nx);
-    return kInf;
+    const TileFit *f = tile_fit(v, zero);
+    return f ? tile_us(v, *f, ny, nx) : kInf;
   }
   if (v.mf == 7) {
     const StripFit *f = by_id(kStrip, v.id);
@@ -172,6 +179,11 @@ double launch_us_2d(const Variant &v, int64_t ny, int64_t nx, bool zero) {
     return f && (zero || v.kf == 1) ? mfma_us(v, *f, ny, nx) : kInf;
   }
   return kInf;
+}
+
+double tiles_us_2d(const Variant &v, int64_t tiles, int64_t edge, double cells) {
+  const TileFit *f = tile_fit(v, true);
+  return f ? tile_us(v, *f, tiles, edge, cells) : kInf;
 }
 
 bool Sequence2D::init(int R, int shape, int64_t ny, int64_t nx, bool zero) {

@@ -8,6 +8,10 @@ namespace cs {
 // +0.  Infinite for a kernel without a prediction or one that the grid does not fit.
 double launch_us_2d(const Variant &v, int64_t ny, int64_t nx, bool zero);
 
+// The same for one launch of a register-tile kernel over the tiles of several grids with +0 halos: `edge` of them
+// in the first or last tile column, `cells` in all grids together.
+double tiles_us_2d(const Variant &v, int64_t tiles, int64_t edge, double cells);
+
 // The launches of any number of steps on one grid, zero halo or not.  Nothing is allocated.
 class Sequence2D {
  public:

@@ -46,6 +46,10 @@ int32_t cs_debug_sequence_2d(int32_t radius, int32_t shape, int64_t ny, int64_t 
 /* The same for 3-D plans with a zero halo on the stacked-wave kernels (steps >= 2). */
 int32_t cs_debug_sequence_3d(int32_t radius, int32_t shape, int64_t nz, int64_t ny, int64_t nx, int64_t steps,
                              int32_t *ids, int64_t *counts, int32_t cap);
+/* Launches on register tiles that an FP64 batch of n grids of one stencil (rows[i] x cols[i], +0 halos) makes for
+ * `steps` steps; 0: it streams them. */
+int32_t cs_debug_batch_tiles(int32_t radius, int32_t shape, int32_t n, const int64_t *rows, const int64_t *cols,
+                             int64_t steps);
 /* k-step table of the 16x16x4 kernels (mf = 16) or the flattened 4x4x4 table of the 1-D kernels'
  * layout (mf = 4): dy[], c0[], live[] (cap entries each); returns the table length, or -1. */
 int32_t cs_debug_ktable(int32_t mf, int32_t radius, int32_t shape, int32_t *dy, int32_t *c0, int32_t *live,

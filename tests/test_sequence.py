@@ -124,3 +124,24 @@ def test_3d_steps(shape):
             assert all(v[0] == shape and v[2] <= n[1] and v[3] <= n[2] and c > 0 for v, c in got)
     assert LIB.cs_debug_sequence_3d(1, shape, 10, 23, 64, 4, ids, counts, 8) == 0
     assert LIB.cs_debug_sequence_3d(2, shape, 100, 100, 100, 4, ids, counts, 8) == 0
+
+
+def _batch_tiles(R, shape, sizes, steps):
+    fn = LIB.cs_debug_batch_tiles
+    fn.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.POINTER(ctypes.c_int64),
+                   ctypes.POINTER(ctypes.c_int64), ctypes.c_int64]
+    col = (ctypes.c_int64 * len(sizes))
+    return fn(R, shape, len(sizes), col(*[s[0] for s in sizes]), col(*[s[1] for s in sizes]), steps)
+
+
+@pytest.mark.parametrize("R,shape,sizes,steps,tiles", [
+    (3, STAR, [(2500, 2500)], 60, False),  # 1029 us on tiles, 864 in strips
+    (3, STAR, [(1200, 1100), (900, 1000), (700, 1400), (1500, 1100)], 60, False),  # 4.7 M cells: 881 / 715
+    (3, STAR, [(900, 1000), (700, 1000), (1000, 1000)], 1, False),  # 94 / 51
+    (3, STAR, [(600, 500)] * 3, 60, True),  # 0.9 M cells: 305 / 620
+    (1, BOX, [(2500, 2500)], 60, True),  # 360 / 526
+    (1, BOX, [(1000, 1000)] * 10, 60, True),  # 10 M cells: 601 / 850
+    (3, STAR, [(63, 300)], 60, False),  # smaller than a tile
+])
+def test_batch_tiles(R, shape, sizes, steps, tiles):
+    assert (_batch_tiles(R, shape, sizes, steps) > 0) == tiles
