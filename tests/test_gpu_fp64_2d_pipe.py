@@ -139,3 +139,36 @@ def test_pipe_variant_alternating_halo(gpu, vid, r, kind, kf, ox, name):
         _check(L, got, want)
         m = ~L.interior_mask()
         assert np.array_equal(got[m], want[m]), runs
+
+
+PIPES = [v for v in VARIANTS if v[5].startswith("k2d_pipe")]
+
+
+@pytest.mark.parametrize("vid,r,kind,kf,ox,name", PIPES, ids=[v[5] for v in PIPES])
+def test_pipe_variant_long_chunks_halo(gpu, vid, r, kind, kf, ox, name):
+    # 40000 rows on two strips: chunks of 150 rows and more, so that the ring of the side halos (64 rows)
+    # wraps and the loop without row checks runs long in the general halo form.  Windows of 1000 rows far from
+    # the first and last row against the oracle on their rows and those that they depend on
+    print(f"case {name} long chunks", flush=True)
+    offs = shape_offsets(f"{kind}2d{r}r")
+    ny, nx, steps = 40000, 512 + ox, 2 * kf
+    L = Layout.with_halo([ny, nx], r)
+    w = oracle.fill_weights(len(offs), vid)
+    x = np.random.default_rng(vid).uniform(-1, 1, L.cells)
+    with Plan(L, r, dense_weights(2, r, offs, w), variant=vid) as p:
+        assert f"variant={vid}" in p.describe()
+        p.upload(x)
+        p.run(steps)
+        got = p.download()
+    n, reach = 1000, r * steps
+    sub = Layout.with_halo([n + 2 * reach, nx], r)
+    pitch = sub.cells // (n + 2 * reach + 2 * r)
+    assert L.cells == (ny + 2 * r) * pitch
+    X, G = x.reshape(-1, pitch), got.reshape(-1, pitch)
+    for row in (700, 20011, ny - 1900):
+        part = X[row - reach : row + n + reach + 2 * r]
+        want = oracle.run(sub, offs, w, np.ascontiguousarray(part).ravel(), steps).reshape(-1, pitch)
+        want = want[r + reach : r + reach + n]
+        have = G[r + row : r + row + n]
+        assert np.abs(have[:, r : r + nx] - want[:, r : r + nx]).max() <= 1e-12 * np.abs(want).max(), row
+        assert np.array_equal(have[:, :r], want[:, :r]) and np.array_equal(have[:, r + nx :], want[:, r + nx :])
