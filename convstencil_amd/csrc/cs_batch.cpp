@@ -27,13 +27,14 @@ namespace {
 // One multi-grid launch of a register-streaming variant.
 struct RegLaunch {
   const cs::Variant *v = nullptr;
-  cs::RegItem *items = nullptr;
+  const cs::RegItem *items = nullptr;  // in the sequence's buffer
   int nitems = 0, flip = 0;
   int chain = 0;  // the launches of one stencil class form a chain (one stream)
 };
 
 struct RegSeq {
   std::vector<RegLaunch> launches;
+  cs::RegItem *items = nullptr;  // of all launches
   std::vector<int> parity_flip;  // per grid: its launches (mod 2)
   int chains = 1;
   hipGraphExec_t graph = nullptr;
@@ -167,8 +168,7 @@ cs_status build_seq(cs_batch *b, int64_t steps, Seq *s) {
 
 void free_rseq(RegSeq &s) {
   if (s.graph) (void)hipGraphExecDestroy(s.graph);
-  for (RegLaunch &l : s.launches)
-    if (l.items) (void)hipFree(l.items);
+  if (s.items) (void)hipFree(s.items);
   s = RegSeq{};
 }
 
@@ -296,35 +296,39 @@ cs_status build_rseq(cs_batch *b, int64_t steps, RegSeq *s) {
     nj = std::max(nj, seq[(size_t)g].size());
     s->parity_flip.push_back((int)(seq[(size_t)g].size() & 1));
   }
-  std::map<std::pair<int, const cs::Variant *>, std::vector<cs::RegItem>> cache;
+  // Launches of one variant over the same grids share one list of items, and all lists one buffer: 500 steps of 24
+  // grids are hundreds of launches of about a dozen lists.
+  typedef std::pair<const cs::Variant *, std::vector<int>> Members;
+  std::map<Members, std::pair<size_t, int>> lists;  // first item, items
+  std::vector<cs::RegItem> items;
+  std::vector<size_t> first;  // per launch
   for (size_t j = 0; j < nj; ++j) {
     // per variant and chain: a chain's launches keep its stream
-    std::map<std::pair<const cs::Variant *, int>, std::vector<cs::RegItem>> groups;
-    for (int g = 0; g < b->count; ++g) {
-      if (j >= seq[(size_t)g].size()) continue;
-      const cs::Variant *v = seq[(size_t)g][j];
-      auto key = std::make_pair(g, v);
-      auto c = cache.find(key);
-      if (c == cache.end()) {
-        std::vector<cs::RegItem> it;
-        reg_items(b, g, v, rows[(size_t)chain[(size_t)g]], &it);
-        c = cache.emplace(key, it).first;
-      }
-      std::vector<cs::RegItem> &dst = groups[std::make_pair(v, launch[(size_t)g])];
-      dst.insert(dst.end(), c->second.begin(), c->second.end());
-    }
+    std::map<std::pair<const cs::Variant *, int>, std::vector<int>> groups;
+    for (int g = 0; g < b->count; ++g)
+      if (j < seq[(size_t)g].size()) groups[std::make_pair(seq[(size_t)g][j], launch[(size_t)g])].push_back(g);
     for (auto &kv : groups) {
-      if (kv.second.empty()) continue;
-      if (kv.second.size() > (size_t)0x7fffffff) return CS_ERR_UNSUPPORTED;
-      RegLaunch l;
-      l.v = kv.first.first;
-      l.nitems = (int)kv.second.size();
-      l.flip = (int)(j & 1);
-      l.chain = kv.first.second;
-      CS_HIP(hipMalloc(&l.items, kv.second.size() * sizeof(cs::RegItem)));
-      s->launches.push_back(l);  // freed with the sequence from here on
-      CS_HIP(hipMemcpy(l.items, kv.second.data(), kv.second.size() * sizeof(cs::RegItem), hipMemcpyHostToDevice));
+      auto l = lists.find(Members(kv.first.first, kv.second));
+      if (l == lists.end()) {
+        const size_t at = items.size();
+        for (int g : kv.second) reg_items(b, g, kv.first.first, rows[(size_t)chain[(size_t)g]], &items);
+        if (items.size() - at > (size_t)0x7fffffff) return CS_ERR_UNSUPPORTED;
+        l = lists.emplace(Members(kv.first.first, kv.second), std::make_pair(at, (int)(items.size() - at))).first;
+      }
+      if (l->second.second == 0) continue;
+      RegLaunch r;
+      r.v = kv.first.first;
+      r.nitems = l->second.second;
+      r.flip = (int)(j & 1);
+      r.chain = kv.first.second;
+      first.push_back(l->second.first);
+      s->launches.push_back(r);
     }
+  }
+  if (!items.empty()) {
+    CS_HIP(hipMalloc(&s->items, items.size() * sizeof(cs::RegItem)));
+    CS_HIP(hipMemcpy(s->items, items.data(), items.size() * sizeof(cs::RegItem), hipMemcpyHostToDevice));
+    for (size_t i = 0; i < first.size(); ++i) s->launches[i].items = s->items + first[i];
   }
   s->chains = (int)classes.size();
   return CS_OK;

@@ -4,12 +4,13 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <utility>
 
 namespace {
-int g_dev = 0, g_launches = 0, g_refused = 0;
+int g_dev = 0, g_launches = 0, g_refused = 0, g_mallocs = 0, g_frees = 0, g_copies = 0;
 std::map<std::pair<int, const void *>, int> g_lds;
 double g_scratch[2][4096];
 hipError_t g_last = hipSuccess;
@@ -23,6 +24,9 @@ struct Call {
 extern "C" {
 int stub_launches() { return g_launches; }
 int stub_refused() { return g_refused; }
+int stub_mallocs() { return g_mallocs; }
+int stub_frees() { return g_frees; }
+int stub_copies() { return g_copies; }
 
 hipError_t hipGetDeviceCount(int *n) { return *n = 2, hipSuccess; }
 hipError_t hipGetDevice(int *d) { return *d = g_dev, hipSuccess; }
@@ -62,5 +66,31 @@ hipError_t hipGetLastError() {
   g_last = hipSuccess;
   return e;
 }
+// device memory is host memory
+hipError_t hipMalloc(void **p, size_t n) {
+  ++g_mallocs;
+  return (*p = calloc(n, 1)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void *p) {
+  g_frees += p != nullptr;
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipMemset(void *p, int v, size_t n) { return memset(p, v, n), hipSuccess; }
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) { return memset(p, v, n), hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
+  ++g_copies;
+  return memcpy(d, s, n), hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = (hipStream_t)&g_call, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { return *e = (hipEvent_t)&g_call, hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stub"; }
 }

@@ -1,5 +1,5 @@
-"""A second device in one process: the large-LDS kernels are prepared on each device that runs them.
-Host code only, on a stub of the HIP runtime in a process of its own."""
+"""Host code on a stub of the HIP runtime, in a process of its own: the large-LDS kernels are prepared on each
+device that runs them; a batch's first run of a step count allocates and copies once."""
 import os
 import shutil
 import subprocess
@@ -45,11 +45,48 @@ sys.exit(1 if bad or stub.stub_refused() or not stub.stub_launches() else 0)
 """
 
 
-@pytest.mark.skipif(not shutil.which("g++") or not os.path.isdir(INCLUDE), reason="needs g++ and the HIP headers")
-def test_kernels_are_prepared_on_every_device(tmp_path):
+BATCH = r"""
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+from convstencil_amd import Batch, Layout, dense_weights, shape_offsets
+items = []
+for shape, r, ny, nx in (("box2d1r", 1, 300, 400), ("box2d1r", 1, 200, 150), ("star2d3r", 3, 500, 300),
+                         ("star2d3r", 3, 300, 200), ("box2d1r", 1, 20, 90)):
+    offs = shape_offsets(shape)
+    items.append((Layout.with_halo([ny, nx], r), r, dense_weights(2, r, offs, np.full(len(offs), 1.0 / len(offs)))))
+with Batch(*zip(*items)) as b:
+    for g, (L, r, w) in enumerate(items):
+        b.upload(g, np.zeros(L.cells))
+    before = stub.stub_mallocs(), stub.stub_copies()
+    n0 = stub.stub_launches()
+    b.run(500)
+    mallocs, copies = stub.stub_mallocs() - before[0], stub.stub_copies() - before[1]
+    launches = stub.stub_launches() - n0
+    print("launches", launches, "allocations", mallocs, "copies", copies)
+    # one buffer with every list of items, one copy into it, one of the grid table and one of the error word
+    ok = launches > 200 and mallocs <= 1 and copies <= 3
+print("allocations", stub.stub_mallocs(), "freed", stub.stub_frees())
+sys.exit(0 if ok and stub.stub_mallocs() == stub.stub_frees() else 1)
+"""
+
+NEEDS = pytest.mark.skipif(not shutil.which("g++") or not os.path.isdir(INCLUDE), reason="needs g++ and the HIP headers")
+
+
+def _run_on_stub(tmp_path, child):
     so = str(tmp_path / "hip_stub.so")
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", INCLUDE,
                     os.path.join(HERE, "hip_stub.cpp"), "-o", so], check=True, timeout=120)
-    p = subprocess.run([sys.executable, "-c", CHILD, so], cwd=os.path.dirname(HERE), capture_output=True, text=True,
+    p = subprocess.run([sys.executable, "-c", child, so], cwd=os.path.dirname(HERE), capture_output=True, text=True,
                        timeout=300)
     assert p.returncode == 0, p.stdout + p.stderr
+
+
+@NEEDS
+def test_kernels_are_prepared_on_every_device(tmp_path):
+    _run_on_stub(tmp_path, CHILD)
+
+
+@NEEDS
+def test_a_batch_uploads_its_launch_lists_at_once(tmp_path):
+    _run_on_stub(tmp_path, BATCH)
