@@ -44,7 +44,7 @@ class Sequence2D {
     if (ones > 0) f(one_, ones);
   }
 
-  // f(variant) for every variant that a number of steps can take.
+  // f(variant) for a variant of every kernel that a number of steps can take (a tile's depths share one).
   template <class F>
   void each_variant(F f) const {
     bool used[kDepths + 1] = {};
@@ -52,10 +52,8 @@ class Sequence2D {
       for (int i = 1; i <= kSteps; ++i) used[(int)pick_[e][i]] = true;
     f(one_);
     f(bulk_);
-    for (int k = 1; k <= kDepths; ++k) {
-      if (used[k] && depth_[k] != bulk_) f(depth_[k]);
-      if (tile_[k] && tile_[k] != depth_[k]) f(tile_[k]);
-    }
+    for (int k = 1; k <= kDepths; ++k)
+      if (used[k] && depth_[k] != bulk_ && depth_[k] != tile_[k]) f(depth_[k]);
   }
 
  private:
