@@ -46,6 +46,8 @@ struct cs_plan {
   const Variant *vmain = nullptr;
   std::vector<const Variant *> vrem;  // vrem[r] runs r fused steps (r < vmain->kf), may be null
   const Variant *vone = nullptr;      // single-step variant (the register families use the MFMA one)
+  const Variant *vzero = nullptr;     // with a zero halo in place of vmain, and its vrem (strip_of)
+  std::vector<const Variant *> vzrem;
   // 2-D FP64 plans that choose for themselves: the sequences for a zero halo [1] and another one [0]
   bool by_time = false;
   cs::Sequence2D seq[2];
@@ -201,6 +203,15 @@ const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t
   return find_variant(2, 10, R, shape, depth, 0);
 }
 
+// With a zero halo the radius-1 box runs faster in register-streaming strips of the same depth where the
+// pipeline's wide strips overlap or are few: measured, us of 48 steps, strips / pipeline, 20000 x 520 418 / 531,
+// 100000 x 520 1562 / 2068, 20000 x 1030 704 / 728, 20000 x 1500 911 / 937, 8000 x 2000 524 / 546, 2300^2 259 /
+// 263, 3500^2 409 / 431, but 4096^2 519 / 510, 2000 x 10000 577 / 552, 8192^2 1728 / 1519.  Else null.
+const Variant *strip_of(const Variant *v, int fusion_depth, int64_t ny, int64_t nx) {
+  if (v->mf != 10 || v->R != 1 || v->shape != cs::SHAPE_BOX || fusion_depth != v->kf) return nullptr;
+  return nx <= 2048 || ny * nx < 15000000 ? find_variant(2, 7, 1, cs::SHAPE_BOX, v->kf, 0) : nullptr;
+}
+
 // The main variant of a plan: a forced id, else the preferred family's default depth (ny x nx = the
 // interior of one grid, 0 when no single grid decides).
 const Variant *pick_main(int nd, int R, int shape, int prec, int fusion_depth, int tile_variant, int64_t ny = 0,
@@ -332,9 +343,17 @@ cs_status select_variants(cs_plan *p) {
   p->vrem.assign(v->kf, nullptr);
   for (int r = 1; r < v->kf && !p->by_time && !p->by_time3; ++r)
     p->vrem[r] = remainder_variant(nd, p->R, p->shape, v, r, prec, fam);
-  for (const Variant *u : {p->vmain, p->vone}) CS_HIP(u->prepare());
-  for (const Variant *u : p->vrem)
+  p->vzero = p->opt.tile_variant <= 0 && prec == CS_PREC_FP64 && nd == 2
+                 ? strip_of(v, p->opt.fusion_depth, p->L.n[1], p->L.n[2])
+                 : nullptr;
+  p->vzrem.clear();
+  for (int r = 0; p->vzero && r < v->kf; ++r)
+    p->vzrem.push_back(r > 0 ? remainder_variant(nd, p->R, p->shape, p->vzero, r, prec, fam) : nullptr);
+  for (const Variant *u : {p->vmain, p->vone, p->vzero})
     if (u) CS_HIP(u->prepare());
+  for (const auto *rem : {&p->vrem, &p->vzrem})
+    for (const Variant *u : *rem)
+      if (u) CS_HIP(u->prepare());
   if (p->by_time) CS_TRY(prepare_sequence(p->seq[1]));
   if (p->by_time3) CS_TRY(prepare_sequence(p->seq3));
   if (prec != CS_PREC_FP64) {
@@ -407,6 +426,8 @@ cs_status launch_one(cs_plan *p, const Variant *v, int64_t done) {
   return CS_OK;
 }
 
+const Variant *main_variant(const cs_plan *p) { return p->halo_uniform && p->vzero ? p->vzero : p->vmain; }
+
 // Whether the plan's launches may fuse steps: with halos that differ between the buffers only
 // the level-pipelined and the register-tile kernels can (they read every level's halo from its
 // own buffer).
@@ -448,12 +469,14 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
     p->seq3.each(steps, [&](const Variant *v, int64_t n) { seq->insert(seq->end(), (size_t)n, v); });
     return;
   }
-  if (!fuses(p) || p->vmain->kf == 1) {
+  const Variant *vmain = main_variant(p);
+  const std::vector<const Variant *> &vrem = vmain == p->vmain ? p->vrem : p->vzrem;
+  if (!fuses(p) || vmain->kf == 1) {
     seq->assign((size_t)steps, p->vone);
     return;
   }
-  const int kf = p->vmain->kf;
-  if (p->opt.precision == CS_PREC_FP64 && (p->vmain->mf == 11 || p->vmain->mf == 12)) {
+  const int kf = vmain->kf;
+  if (p->opt.precision == CS_PREC_FP64 && (vmain->mf == 11 || vmain->mf == 12)) {
     // every depth is compiled (mf 12: from 2 up): as few launches as the main depth allows, cut
     // evenly.  With halos that differ an odd number of even depths k has one of them cut into k - 1
     // and 1.
@@ -461,33 +484,33 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
     int64_t even = 0;
     for (int64_t i = 0; i < n; ++i) {
       const int64_t d = steps / n + (i < steps % n);
-      const Variant *u = d == kf ? p->vmain : p->vrem[(size_t)d];
+      const Variant *u = d == kf ? vmain : vrem[(size_t)d];
       seq->push_back(u ? u : p->vone);
       even += d % 2 == 0;
     }
     if (!p->halo_uniform && even % 2) {
       size_t i = 0;
       while ((*seq)[i]->kf % 2) ++i;
-      (*seq)[i] = p->vrem[(size_t)(*seq)[i]->kf - 1];
+      (*seq)[i] = vrem[(size_t)(*seq)[i]->kf - 1];
       seq->push_back(p->vone);
     }
     return;
   }
-  seq->assign((size_t)(steps / kf), p->vmain);
+  seq->assign((size_t)(steps / kf), vmain);
   int64_t rem = steps % kf;
   while (rem > 0) {
     const Variant *best = p->vone;
-    for (const Variant *u : p->vrem)
+    for (const Variant *u : vrem)
       if (u && u->kf <= rem && u->kf > best->kf && (p->halo_uniform || u->mf == 10)) best = u;
     seq->push_back(best);
     rem -= best->kf;
   }
-  if (p->opt.precision == CS_PREC_FP64 && p->vmain->mf == 10 && steps > kf && steps % kf) {
+  if (p->opt.precision == CS_PREC_FP64 && vmain->mf == 10 && steps > kf && steps % kf) {
     // a shallow last launch moves as many bytes as a deep one: kf + r steps are better cut
     // evenly (box r1 10240^2, 12 + 4 against 8 + 8 steps: 0.91 against 0.84 ms)
     const int r = (int)(steps % kf);
     for (int b = (kf + r) / 2; b > r; --b) {
-      const Variant *u = kf + r - b < kf ? p->vrem[(size_t)(kf + r - b)] : nullptr, *v = p->vrem[(size_t)b];
+      const Variant *u = kf + r - b < kf ? vrem[(size_t)(kf + r - b)] : nullptr, *v = vrem[(size_t)b];
       if (!u || !v || (!p->halo_uniform && (u->mf != 10 || v->mf != 10))) continue;
       seq->resize((size_t)(steps / kf) - 1);
       seq->push_back(u);
@@ -502,7 +525,7 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
   for (size_t i = n; i-- > 0;) {
     const int k = (*seq)[i]->kf;
     for (int half = k / 2; half >= 1; --half) {
-      const Variant *u = p->vrem[(size_t)half], *v = p->vrem[(size_t)(k - half)];
+      const Variant *u = vrem[(size_t)half], *v = vrem[(size_t)(k - half)];
       if (!u || !v || u->mf != 10 || v->mf != 10) continue;
       (*seq)[i] = v;
       seq->insert(seq->begin() + (ptrdiff_t)n, u);
@@ -815,6 +838,7 @@ cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int t
                              const Variant **vmain, const Variant **vone, const Variant **vrem, int vrem_cap) {
   const Variant *v = pick_main(ndim, R, shape, CS_PREC_FP64, fusion_depth, tile_variant, ny, nx);
   if (!v) return tile_variant > 0 ? CS_ERR_INVALID : CS_ERR_UNSUPPORTED;
+  if (const Variant *u = tile_variant <= 0 && ndim == 2 ? strip_of(v, fusion_depth, ny, nx) : nullptr) v = u;
   if (v->kf > vrem_cap) return CS_ERR_UNSUPPORTED;
   *vmain = v;
   *vone = single_step(ndim, R, v->shape, v);
@@ -967,7 +991,7 @@ cs_status cs_plan_run(cs_plan *p, int64_t steps, cs_report *rep) {
     memset(rep, 0, sizeof(*rep));
     rep->launches = p->launches - l0;
     rep->fusion_depth = executed_depth(p, steps);
-    rep->variant = p->vmain->id;
+    rep->variant = main_variant(p)->id;
   }
   return CS_OK;
 }
@@ -1000,7 +1024,7 @@ cs_status cs_plan_time(cs_plan *p, int64_t steps, int32_t warmup, int32_t reps, 
     rep->gstencil_per_s = rep->elapsed_ms > 0 && pts > 0 ? pts * (double)steps / (rep->elapsed_ms * 1e-3) / 1e9 : 0.0;
     rep->launches = (p->launches - l0) / reps;
     rep->fusion_depth = executed_depth(p, steps);
-    rep->variant = p->vmain->id;
+    rep->variant = main_variant(p)->id;
   }
   return CS_OK;
 }
@@ -1030,10 +1054,11 @@ cs_status cs_plan_device_buffers(cs_plan *p, double **current, double **other) {
 cs_status cs_plan_describe(cs_plan *p, char *buf, int32_t len) {
   if (!p || !buf || len <= 0) return CS_ERR_INVALID;
   static const char *how[3] = {"default", "cached", "timed"};
+  const Variant *v = main_variant(p);
   snprintf(buf, (size_t)len,
            "variant=%d name=%s mf=%d R=%d shape=%s kf=%d tile=%dx%d waves=%d lds=%zu halo_uniform=%d autotune=%s",
-           p->vmain->id, p->vmain->name, p->vmain->mf, p->R, p->shape == cs::SHAPE_BOX ? "box" : "star", p->vmain->kf,
-           p->vmain->by, p->vmain->bx, p->vmain->nw, p->vmain->lds_bytes, (int)p->halo_uniform, how[p->tuned]);
+           v->id, v->name, v->mf, p->R, p->shape == cs::SHAPE_BOX ? "box" : "star", v->kf, v->by, v->bx, v->nw, v->lds_bytes,
+           (int)p->halo_uniform, how[p->tuned]);
   return CS_OK;
 }
 
@@ -1059,7 +1084,7 @@ cs_status cs_run(const cs_layout *layout, const cs_stencil *st, const double *ho
     rep->gstencil_per_s = ms > 0 ? pts * (double)steps / (ms * 1e-3) / 1e9 : 0.0;
     rep->launches = p->launches - l0;
     rep->fusion_depth = executed_depth(p, steps);
-    rep->variant = p->vmain->id;
+    rep->variant = main_variant(p)->id;
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);

@@ -172,3 +172,24 @@ def test_pipe_variant_long_chunks_halo(gpu, vid, r, kind, kf, ox, name):
         have = G[r + row : r + row + n]
         assert np.abs(have[:, r : r + nx] - want[:, r : r + nx]).max() <= 1e-12 * np.abs(want).max(), row
         assert np.array_equal(have[:, :r], want[:, :r]) and np.array_equal(have[:, r + nx :], want[:, r + nx :])
+
+
+@pytest.mark.parametrize("ny,nx,strips", [(9700, 520, True), (2300, 2300, True), (2000, 7600, False)])
+def test_depth_12_box_by_halo(gpu, ny, nx, strips):
+    # depth 12 asked for, the radius-1 box: strips of that depth with a zero halo where they are faster (10000 x 520,
+    # 48 steps, 281 us against the pipeline's 348), the pipeline with an uploaded halo
+    print(f"case depth 12 {ny}x{nx}", flush=True)
+    offs = shape_offsets("box2d1r")
+    L = Layout.with_halo([ny, nx], 1)
+    w = oracle.fill_weights(len(offs), ny)
+    zero = oracle.fill_data(L, ny)
+    halo = np.random.default_rng(ny).uniform(-1, 1, L.cells)
+    with Plan(L, 1, dense_weights(2, 1, offs, w), fusion_depth=12) as p:
+        for x in (zero, halo, zero):
+            p.upload(x)
+            family = "k2d_reg" if strips and x is zero else "k2d_pipe"
+            assert f"name={family}" in p.describe()
+            for s in (12, 24, 11):
+                p.run(s)
+            got = p.download()
+            _check(L, got, oracle.run(L, offs, w, x, 47))
