@@ -145,14 +145,14 @@ int max_kf(int ndim, int mf, int R, int shape, int prec = CS_PREC_FP64, int st =
 // first single-step variant -- except that the register kernels' single steps (alternating
 // halos, remainders of one step) run on the LDS-staged MFMA single-step kernel, which keeps
 // more bytes in flight: measured (GStencil/s) box2d1r 10240^2 300 against 203, star2d3r
-// 8192^2 286 against 253; box2d3r keeps its own (246 against 204).
+// 8192^2 286 against 253, box2d3r 204 against 133 (1024^2 117 against 15).
 const Variant *single_step(int nd, int R, int shape, const Variant *v) {
   if (v->kf == 1) return v;
   // the fused 3-D register and tile kernels: the 8 x 8 block single-step kernel (512^3: 258-268
   // GStencil/s against 242 for the register single step)
   if ((v->mf == 9 || v->mf == 12) && nd == 3)
     if (const Variant *m = find_variant(nd, 8, R, shape, 1, 0, CS_PREC_FP64)) return m;
-  if ((v->mf == 6 || v->mf == 7 || v->mf == 10) && !(nd == 2 && R > 1 && shape == cs::SHAPE_BOX))
+  if (v->mf == 10 || ((v->mf == 6 || v->mf == 7) && !(nd == 2 && R > 1 && shape == cs::SHAPE_BOX)))
     if (const Variant *m = find_variant(nd, 4, R, shape, 1, 0, CS_PREC_FP64)) return m;
   if (v->mf == 10) return find_variant(nd, 7, R, shape, 1, 0, CS_PREC_FP64);
   if (v->mf == 11) return find_variant(nd, 11, R, shape, 1, 0, CS_PREC_FP64, v->st);
@@ -173,8 +173,8 @@ bool fits(const Variant *v, int64_t ny, int64_t nx) {
 
 // The variant that runs r steps left over by a main variant v; null where there is none.  The
 // level-pipelined kernels are compiled for a few depths only; the register-streaming kernels
-// fill in, except for the radius-3 box, where those spill (3 steps at once 195 GStencil/s, 2 + 1
-// steps 320).
+// fill in, for the radius-3 box, where those spill, the dilated tables (3 steps of 4096^2 171 us, as
+// 2 + 1 188).
 const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int r, int prec, int st) {
   if (prec == CS_PREC_FP64 && v->mf == 12) {  // the same tile's shallower variants
     int cnt = 0;
@@ -186,8 +186,8 @@ const Variant *remainder_variant(int nd, int R, int shape, const Variant *v, int
   if (prec != CS_PREC_FP64 && v->st == 3)  // the bits of depth 2: even depths, with its anchors above it
     return r > 1 && r % 2 ? nullptr : find_variant(nd, v->mf, R, shape, r, 0, prec, r > 2 ? 3 : 2);
   const Variant *u = find_variant(nd, v->mf, R, shape, r, 0, prec, v->mf == 11 && prec == CS_PREC_FP64 ? v->st : st);
-  if (!u && prec == CS_PREC_FP64 && v->mf == 10 && !(R > 1 && shape == cs::SHAPE_BOX))
-    u = find_variant(nd, 7, R, shape, r, 0, prec);
+  if (!u && prec == CS_PREC_FP64 && v->mf == 10)
+    u = find_variant(nd, R > 1 && shape == cs::SHAPE_BOX ? 4 : 7, R, shape, r, 0, prec);
   return u;
 }
 
@@ -511,7 +511,7 @@ void plan_sequence(const cs_plan *p, int64_t steps, std::vector<const Variant *>
     const int r = (int)(steps % kf);
     for (int b = (kf + r) / 2; b > r; --b) {
       const Variant *u = kf + r - b < kf ? vrem[(size_t)(kf + r - b)] : nullptr, *v = vrem[(size_t)b];
-      if (!u || !v || (!p->halo_uniform && (u->mf != 10 || v->mf != 10))) continue;
+      if (!u || !v || u->mf == 4 || (!p->halo_uniform && (u->mf != 10 || v->mf != 10))) continue;
       seq->resize((size_t)(steps / kf) - 1);
       seq->push_back(u);
       seq->push_back(v);
@@ -762,13 +762,9 @@ cs_status autotune_plan(cs_plan *p, int classified) {
 
 namespace cs {
 
-// The FP64 kernel choice of a plan, made without a plan (nothing allocated, no device
-// touched): the main variant, the single-step variant and one variant per remainder depth
-// 1 .. kf - 1 (vrem[r], null where the family has none), as select_variants picks them for
-// a grid of ny x nx interior cells.
-// The launch sequence of the register-streaming 2-D family for `steps` steps of a radius-R
-// stencil of this shape class: the plan's default depth as often as it fits, then the
-// family's largest depth that fits the rest; empty when the plan would not take the family.
+// A batch's launches of the register-streaming 2-D family for `steps` steps of a radius-R
+// stencil of this shape class: the family's default depth as often as it fits, then its
+// largest depth that fits the rest; empty where it has none.
 void reg_sequence(int R, int shape, int64_t steps, std::vector<const Variant *> *seq) {
   seq->clear();
   const Variant *v = pick_main(2, R, shape, CS_PREC_FP64, 0, 0);  // no single grid: never mf 10
@@ -834,6 +830,10 @@ cs_status block_sequence(int R, int shape, const std::vector<std::pair<int64_t, 
   return CS_OK;
 }
 
+// The FP64 kernel choice of a plan with a depth or a variant of its caller's, made without a plan (nothing
+// allocated, no device touched): the main variant, the single-step variant and one variant per
+// remainder depth 1 .. kf - 1 (vrem[r], null where the family has none), as select_variants picks them
+// for a grid of ny x nx interior cells with a zero halo.
 cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int tile_variant, int64_t ny, int64_t nx,
                              const Variant **vmain, const Variant **vone, const Variant **vrem, int vrem_cap) {
   const Variant *v = pick_main(ndim, R, shape, CS_PREC_FP64, fusion_depth, tile_variant, ny, nx);
