@@ -205,11 +205,18 @@ const Variant *pick_pipe(int R, int shape, int fusion_depth, int64_t ny, int64_t
 
 // With a zero halo the radius-1 box runs faster in register-streaming strips of the same depth where the
 // pipeline's wide strips overlap or are few: measured, us of 48 steps, strips / pipeline, 20000 x 520 418 / 531,
-// 100000 x 520 1562 / 2068, 20000 x 1030 704 / 728, 20000 x 1500 911 / 937, 8000 x 2000 524 / 546, 2300^2 259 /
-// 263, 3500^2 409 / 431, but 4096^2 519 / 510, 2000 x 10000 577 / 552, 8192^2 1728 / 1519.  Else null.
+// 100000 x 520 1562 / 2068, 30000 x 1030 988 / 1031, 3000^2 315 / 360, 5000 x 2000 356 / 385, 3500^2 409 / 431, but
+// 2300^2 260 / 259, 3600 x 4400 495 / 454, 12000 x 1500 597 / 604 (17 steps 291 / 275), 8192^2 1728 / 1519.  Else null.
 const Variant *strip_of(const Variant *v, int fusion_depth, int64_t ny, int64_t nx) {
   if (v->mf != 10 || v->R != 1 || v->shape != cs::SHAPE_BOX || fusion_depth != v->kf) return nullptr;
-  return nx <= 2048 || ny * nx < 15000000 ? find_variant(2, 7, 1, cs::SHAPE_BOX, v->kf, 0) : nullptr;
+  const int64_t cells = ny * nx;
+  return nx <= 1100 || (cells >= 6000000 && cells < 13000000) ? find_variant(2, 7, 1, cs::SHAPE_BOX, v->kf, 0) : nullptr;
+}
+
+// Its r steps left over: eight in the pipeline (5000 x 2000 59 us, in strips 80; 20000 x 520 92, 96).
+const Variant *strip_remainder(const Variant *strip, int r) {
+  return r == 8 ? find_variant(2, 10, 1, cs::SHAPE_BOX, 8, 0)
+                : remainder_variant(2, 1, cs::SHAPE_BOX, strip, r, CS_PREC_FP64, -1);
 }
 
 // The main variant of a plan: a forced id, else the preferred family's default depth (ny x nx = the
@@ -348,7 +355,7 @@ cs_status select_variants(cs_plan *p) {
                  : nullptr;
   p->vzrem.clear();
   for (int r = 0; p->vzero && r < v->kf; ++r)
-    p->vzrem.push_back(r > 0 ? remainder_variant(nd, p->R, p->shape, p->vzero, r, prec, fam) : nullptr);
+    p->vzrem.push_back(r > 0 ? strip_remainder(p->vzero, r) : nullptr);
   for (const Variant *u : {p->vmain, p->vone, p->vzero})
     if (u) CS_HIP(u->prepare());
   for (const auto *rem : {&p->vrem, &p->vzrem})
@@ -838,13 +845,16 @@ cs_status pick_fp64_variants(int ndim, int R, int shape, int fusion_depth, int t
                              const Variant **vmain, const Variant **vone, const Variant **vrem, int vrem_cap) {
   const Variant *v = pick_main(ndim, R, shape, CS_PREC_FP64, fusion_depth, tile_variant, ny, nx);
   if (!v) return tile_variant > 0 ? CS_ERR_INVALID : CS_ERR_UNSUPPORTED;
-  if (const Variant *u = tile_variant <= 0 && ndim == 2 ? strip_of(v, fusion_depth, ny, nx) : nullptr) v = u;
+  const Variant *strip = tile_variant <= 0 && ndim == 2 ? strip_of(v, fusion_depth, ny, nx) : nullptr;
+  if (strip) v = strip;
   if (v->kf > vrem_cap) return CS_ERR_UNSUPPORTED;
   *vmain = v;
   *vone = single_step(ndim, R, v->shape, v);
   if (!*vone) return CS_ERR_UNSUPPORTED;
   for (int r = 0; r < vrem_cap; ++r)
-    vrem[r] = r >= 1 && r < v->kf ? remainder_variant(ndim, R, v->shape, v, r, CS_PREC_FP64, -1) : nullptr;
+    vrem[r] = r < 1 || r >= v->kf ? nullptr
+              : strip             ? strip_remainder(strip, r)
+                                  : remainder_variant(ndim, R, v->shape, v, r, CS_PREC_FP64, -1);
   return CS_OK;
 }
 

@@ -174,7 +174,7 @@ def test_pipe_variant_long_chunks_halo(gpu, vid, r, kind, kf, ox, name):
         assert np.array_equal(have[:, :r], want[:, :r]) and np.array_equal(have[:, r + nx :], want[:, r + nx :])
 
 
-@pytest.mark.parametrize("ny,nx,strips", [(9700, 520, True), (2300, 2300, True), (2000, 7600, False)])
+@pytest.mark.parametrize("ny,nx,strips", [(9700, 520, True), (2600, 2500, True), (2000, 7600, False)])
 def test_depth_12_box_by_halo(gpu, ny, nx, strips):
     # depth 12 asked for, the radius-1 box: strips of that depth with a zero halo where they are faster (10000 x 520,
     # 48 steps, 281 us against the pipeline's 348), the pipeline with an uploaded halo
@@ -189,7 +189,7 @@ def test_depth_12_box_by_halo(gpu, ny, nx, strips):
             p.upload(x)
             family = "k2d_reg" if strips and x is zero else "k2d_pipe"
             assert f"name={family}" in p.describe()
-            for s in (12, 24, 11):
+            for s in (12, 20, 11):
                 p.run(s)
             got = p.download()
-            _check(L, got, oracle.run(L, offs, w, x, 47))
+            _check(L, got, oracle.run(L, offs, w, x, 43))
