@@ -127,7 +127,7 @@ class Plan:
 
 
 class Batch:
-    """Many independent 2-D grids advanced together by one persistent launch per run
+    """Many independent 2-D grids advanced together, in launches that they share
     (cs_batch_*): each grid has its own layout, radius and weights."""
 
     def __init__(self, layouts, radii, weights_dense, precision="fp64", use_graph=False):

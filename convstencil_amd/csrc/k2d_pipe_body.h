@@ -11,13 +11,14 @@
 // levels of 8 columns per lane: 512-column strips at 12 (box radius 1), 16 (star radius 1), 8
 // (star radius 3) or 4 (box radius 3) steps per launch.
 //
-// What bounds them: the FP64 FMA issue and the power it draws.  Of the box radius-1 kernel's
-// vector instructions 94% are FMAs (lane shifts 5%), and its clock falls to 1.82-1.92 GHz on
-// random data against 2.36 GHz on zeros, where the same cycles take 0.45 instead of 0.57 ms
-// (10240^2, depth 12); so what is left to gain is work not done: recomputed rows and columns
-// (11%) and bytes.  Measured, GStencil/s of the kernel alone, k2d_reg / k2d_f64 before and
-// this kernel: box2d1r 10240^2 2037 -> 2280, star2d1r 10240^2 2140 -> 3440, star2d3r 8192^2
-// 1013 -> 1208, box2d3r 8192^2 306 -> 458.
+// What bounds them (profiles/fp64_pipe_tile_counters.md): the boxes FP64 issue and the power it draws.
+// Vector instructions take 81% (radius 1) and 83% (radius 3) of the cycles, 91% and 96% of them are FMAs
+// and multiplications, and the clock falls to 1.7-1.95 GHz on random data against 2.36 GHz on zeros, where the
+// same cycles take 0.45 instead of 0.57 ms (10240^2, depth 12); so what is left to gain is work not done: recomputed
+// rows and columns (11%).  The radius-3 star issues in 61% of the cycles (2.0 GHz): its one workgroup of eight waves
+// per CU meets at a barrier every two rows with no other one to fill the waits.  HBM carries 2.1-3.2 TB/s.
+// Measured, GStencil/s of the kernel alone, k2d_reg / k2d_f64 before and this kernel: box2d1r 10240^2 2037 ->
+// 2280, star2d1r 10240^2 2140 -> 3440, star2d3r 8192^2 1013 -> 1208, box2d3r 8192^2 306 -> 458.
 //
 // Rows.  A wave's level s keeps partial sums for the 2R + 1 rows that the incoming row
 // contributes to, as in k2d_reg.hip; the sum order per output is the same (rows dy = -R .. R,

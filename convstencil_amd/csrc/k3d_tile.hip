@@ -16,9 +16,10 @@
 // lane shifts' missing sources (zero), shared rows that are never written (zero) and planes
 // that are set to zero; no row or column is masked.
 //
-// What bounds them: 512^3 box, depth 4: FP64 issue (a 27-tap row costs 27 FMAs and 5 lane-shift
-// moves a cell; 1.27 times the cells for the overlap, 53 TFLOP/s of issue); star, depth 4: memory, 4.9
-// TB/s with the overlap's reads; small grids: the launch and the chain of planes.  Measured, us
+// What bounds them (profiles/fp64_pipe_tile_counters.md): 512^3 box, 80 x 64 tiles at depth 3: FP64 issue (87% of
+// the cycles, 43 TFLOP/s; a 27-tap row costs 27 FMAs and 5 lane-shift moves a cell, the overlap 1.19
+// times the cells of a plane); star, 64 x 64 at depth 4: memory, 5.1 TB/s with the overlap's reads; small grids: the
+// launch and the chain of planes.  Measured, us
 // per step, k3d_reg's choice before and now: box 512^3 307 -> 211, 389 x 301 x 517 160 -> 105, 256^3
 // 48 -> 41, 100^3 23.0 -> 8.4, 600 x 64 x 64 19.9 -> 10.9; star 512^3 211 -> 115, 389 x 301 x 517
 // 92 -> 66, 256^3 30.7 -> 23.3, 100^3 11.1 -> 5.9.  Load rings of 2 or 3 planes instead of 1 gave nothing

@@ -134,11 +134,11 @@ cs_status cs_plan_device_buffers(cs_plan *plan, double **current, double **other
 /* Human-readable description of the kernel choice (variant, tile, fusion depth). */
 cs_status cs_plan_describe(cs_plan *plan, char *buf, int32_t len);
 
-/* ---- batches: many independent 2-D grids advanced by one persistent launch ----
+/* ---- batches: many independent 2-D grids advanced together ----
  * No counterpart in the reference (one grid per process).  Every grid has its own
  * layout and stencil; supported stencils are the radius-1 box (box2d1r) and the
  * radius-3 star (star2d3r), in FP64, CS_PREC_BF16X3 and CS_PREC_FP16X2.  cs_batch_run advances every grid by
- * `steps` steps with a single persistent kernel launch (plus a small reset kernel),
+ * `steps` steps, in launches that many grids share or in a single persistent one,
  * optionally captured in a hipGraph (opt->use_graph). */
 typedef struct cs_batch cs_batch;
 cs_status cs_batch_create(cs_batch **batch, int32_t count, const cs_layout *layouts, const cs_stencil *stencils,
@@ -148,9 +148,11 @@ cs_status cs_batch_upload(cs_batch *batch, int32_t grid, const double *host_in);
 /* Seeds grid i with seeds[i] (as cs_plan_fill_random). */
 cs_status cs_batch_fill_random(cs_batch *batch, const uint64_t *seeds);
 /* FP64 batches whose grids all carry a uniform halo advance by multi-grid launches of the
- * register-streaming kernels; the others by one persistent launch, which needs every
- * workgroup resident at once and whose grid-wide barriers wait a bounded time.  A barrier that times out sets the batch's sticky error word: that run,
- * and every later cs_batch_run / cs_batch_time / cs_batch_download of this batch, returns
+ * register-tile or the register-streaming kernels, whichever is predicted to be faster for the grids of a
+ * stencil, and the two stencils' launches run on streams of their own that join the batch's before the run
+ * ends; the others by one persistent launch (plus a small reset kernel), which needs every
+ * workgroup resident at once and whose grid-wide barriers wait a bounded time.  A barrier that times out sets the
+ * batch's sticky error word: that run, and every later cs_batch_run / cs_batch_time / cs_batch_download of this batch, returns
  * CS_ERR_DEVICE (the grids' contents are undefined from then on). */
 cs_status cs_batch_run(cs_batch *batch, int64_t steps, cs_report *report);
 cs_status cs_batch_time(cs_batch *batch, int64_t steps, int32_t warmup, int32_t reps, cs_report *report);
@@ -159,8 +161,8 @@ cs_status cs_batch_describe(cs_batch *batch, char *buf, int32_t len);
 
 /* ---- autotuner cache ----
  * No counterpart in the reference (fixed tiles).  A plan created with autotune times the
- * fitting variants for 24 steps on its own buffers (before any data is uploaded) and keeps
- * the fastest; choices are cached per key "d<ndim>_r<radius>_s<shape>_p<precision>_n<nz>x
+ * fitting variants for at least 96 steps on its own buffers (before any data is uploaded) and keeps
+ * the fastest if it beats the default by 3%; choices are cached per key "d<ndim>_r<radius>_s<shape>_p<precision>_n<nz>x
  * <ny>x<nx>_g<graph>" in memory and in a text file: $CONVSTENCIL_TUNE_CACHE (empty: memory
  * only), else $XDG_CACHE_HOME/convstencil_amd/tune.txt, else $HOME/.cache/convstencil_amd/tune.txt. */
 const char *cs_tune_cache_path(void);
